@@ -131,6 +131,42 @@ def test_qmm_split_k(cuda, bits):
     # 6 output tiles, 32 chunks: K split 8 ways, partial tiles summed in order
     run_case(300, 512, 2048, 64, bits, seed=bits + 77)
 
+def run_bounded(M, N, K, gs, bits, seed):
+    """A prefill product against the f64 one, elementwise within what its
+    roundings allow: each weight s*q + b rounds once to bf16 (2^-9 relative)
+    and the products add up in f32 (at most K 2^-24 of their magnitudes, below
+    2^-11 here), so |err| <= (2^-9 + 2^-11) sum |x w| + 1/2 ulp_bf16(y)."""
+    print(f"[case] M={M} N={N} K={K} gs={gs} bits={bits}", flush=True)
+    w, s, b = synthetic_linear(N, K, gs, bits, seed, scale_dtype=orc.BF16)
+    xb = synthetic_x(M, K, seed + 1)
+    y = host_f32(quantized_matmul(dev_bf16(xb), dev_words(w), dev_bf16(s), dev_bf16(b), transpose=True, group_size=gs,
+                                  bits=bits)).astype(np.float64)
+    x = orc.bf16_bits_to_f32(xb).astype(np.float64)
+    W = orc.affine_dequant_f32(w, s, b, orc.BF16, N, K, gs, bits).reshape(N, K).astype(np.float64)
+    ref = x @ W.T
+    bound = (2.0 ** -9 + 2.0 ** -11) * (np.abs(x) @ np.abs(W).T) + 2.0 ** -9 * np.maximum(np.abs(y), np.abs(ref))
+    worst = float((np.abs(y - ref) / bound).max())
+    assert worst <= 1.0, f"max err / bound = {worst:.3f}"
+
+
+# Windows of scales and biases (whole words: K / group even) and per-step
+# parameter loads (K / group odd); 1, 2, 3, 4, 5 and 9 steps of two 64-wide
+# chunks, odd chunk counts among them; columns that end inside a tile.
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs,K", [(16, 64), (32, 64), (32, 576), (64, 64), (64, 192), (64, 256), (64, 384), (64, 1088),
+                                  (128, 128), (128, 384), (128, 512), (128, 1152)])
+@pytest.mark.parametrize("M,N", [(130, 128), (1029, 5760)])
+def test_qmm_steps_and_windows(cuda, bits, gs, K, M, N):
+    run_bounded(M, N, K, gs, bits, seed=K + gs + bits)
+
+
+# Split K on the small tiles: the splits of group 128 start at whole windows.
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,N,K", [(33, 256, 4096), (97, 512, 8320)])
+def test_qmm_split_k_groups(cuda, bits, gs, M, N, K):
+    run_bounded(M, N, K, gs, bits, seed=M + gs + bits)
+
 
 @pytest.mark.parametrize("xdt", [orc.F32, orc.F16])
 @pytest.mark.parametrize("M", [1, 33])
