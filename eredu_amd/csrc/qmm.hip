@@ -239,30 +239,46 @@ __device__ __forceinline__ int lower_bound_i32(const int32_t* __restrict__ a, in
     return lo;
 }
 
-// Sorted expert indices -> the grouped tile list: expert e owns rows
-// [lower_bound(e), lower_bound(e + 1)) and takes ceil(rows / kBM) entries
-// {e, first, rows, kBM t}.  One workgroup of 1024 threads, experts in passes
-// of 1024 with a block scan of the entry counts; entries at or past `cap`
-// are dropped and the list's remaining entries are marked unused.
-__global__ __launch_bounds__(1024) void qmm_group_tiles(int4* __restrict__ out, const int32_t* __restrict__ rhs,
-                                                        int batch, int experts, int cap) {
+// Prepares a grouped launch.  Workgroup 0: sorted expert indices -> the tile
+// list; expert e owns rows [lower_bound(e), lower_bound(e + 1)) and takes
+// ceil(rows / bm) entries {e, first, rows, bm t}, experts in passes of 1024
+// with a block scan of the entry counts; entries at or past `cap` are dropped
+// and the list's remaining entries are marked unused.  The indices are searched
+// in LDS where they fit (from memory a search is a chain of a dozen trips).
+// The other workgroups meanwhile clear y (rows of no expert stay zero), n bf16
+// values, n a multiple of 4, y 8-byte aligned.
+constexpr int kGroupIds = 8192;
+__global__ __launch_bounds__(1024) void qmm_group_prepare(int4* __restrict__ out, const int32_t* __restrict__ rhs,
+                                                          int batch, int experts, int cap, int bm,
+                                                          uint16_t* __restrict__ y, int64_t n) {
+    if (blockIdx.x > 0) {
+        const int64_t stride = int64_t(gridDim.x - 1) * 4096;
+        for (int64_t i = (int64_t(blockIdx.x - 1) * 1024 + threadIdx.x) * 4; i < n; i += stride)
+            *reinterpret_cast<uint2*>(y + i) = make_uint2(0, 0);
+        return;
+    }
+    __shared__ int32_t ids[kGroupIds];
     __shared__ int scan[1024];
     __shared__ int carry;
     const int tid = threadIdx.x;
+    const bool local = batch <= kGroupIds;
+    if (local)
+        for (int i = tid; i < batch; i += 1024) ids[i] = rhs[i];
     if (tid == 0) carry = 0;
     __syncthreads();
+    const int32_t* search = local ? ids : rhs;
     for (int e0 = 0; e0 < experts; e0 += 1024) {
         const int e = e0 + tid;
         int first = 0, rows = 0;
         if (e < experts) {
-            first = lower_bound_i32(rhs, batch, e);
-            const int end = lower_bound_i32(rhs, batch, e + 1);
+            first = lower_bound_i32(search, batch, e);
+            const int end = lower_bound_i32(search, batch, e + 1);
             rows = end > first ? end - first : 0;
         }
-        const int nt = (rows + kBM - 1) / kBM;
+        const int nt = (rows + bm - 1) / bm;
         scan[tid] = nt;
         __syncthreads();
-        for (int o = 1; o < 1024; o <<= 1) {  // inclusive scan
+        for (int o = 1; o < 1024 && o < experts - e0; o <<= 1) {  // inclusive scan
             const int v = tid >= o ? scan[tid - o] : 0;
             __syncthreads();
             scan[tid] += v;
@@ -270,9 +286,10 @@ __global__ __launch_bounds__(1024) void qmm_group_tiles(int4* __restrict__ out, 
         }
         const int base = carry + scan[tid] - nt;
         for (int t = 0; t < nt; t++)
-            if (base + t < cap) out[base + t] = make_int4(e, first, rows, t * kBM);
+            if (base + t < cap) out[base + t] = make_int4(e, first, rows, t * bm);
+        const int last = experts - e0 < 1024 ? experts - e0 - 1 : 1023;
         __syncthreads();
-        if (tid == 1023) carry += scan[1023];
+        if (tid == last) carry += scan[last];
         __syncthreads();
     }
     for (int i = carry + tid; i < cap; i += 1024) out[i] = make_int4(-1, 0, 0, 0);
@@ -290,33 +307,39 @@ __global__ __launch_bounds__(256) void qmm_gather_rows(uint16_t* __restrict__ xg
     for (int i = threadIdx.x; i < K / 8; i += 256) dst[i] = ok ? from[i] : make_uint4(0, 0, 0, 0);
 }
 
-// y = 0 (n bf16 values, n a multiple of 4, y 8-byte aligned).
-__global__ __launch_bounds__(256) void qmm_zero(uint16_t* __restrict__ y, int64_t n) {
-    for (int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4; i < n; i += int64_t(gridDim.x) * 1024)
-        *reinterpret_cast<uint2*>(y + i) = make_uint2(0, 0);
-}
-
 static bool launch_qmm_grouped_t(const QmmTypes& t, uint16_t* y, const uint16_t* x, const uint32_t* w, const void* s, const void* b,
                                  const int32_t* lhs, const int32_t* rhs, int batch, int64_t x_batches, int experts,
                                  int N, int K, hipStream_t st, const WsSource* src = nullptr) {
-    const int cap = experts + (batch + kBM - 1) / kBM;  // sum over experts of ceil(rows / kBM)
-    // one launch with 32-bit offsets: each expert's codes and the gathered rows below 2^31 bytes
+    // Tiles by the mean number of rows per expert: 64 x 128 up to 96 (two such
+    // workgroups share a CU), 128 x 256 above.  Measured, the SwiGLU of a prompt's
+    // sorted routes, 64 x 128 against 128 x 256 tiles: 128 experts of 768 x 2048 at
+    // 4 rows each 148 / 197 us, at 32 rows 218 / 236, 64 experts of 1024 x 2048 at
+    // 64 rows 178 / 209, at 128 rows 273 / 271; 8 experts of 7168 x 4096 at 128 rows
+    // 408 / 372.  (With 128 x 256 tiles, y cleared and the rows gathered by launches
+    // of their own and the indices searched in memory, before: 276 us at 32 rows.)
+    const int mean = batch / (experts > 0 ? experts : 1);
+    const int tm = mean <= 96 ? 2 : 4, tn = mean <= 96 ? 1 : 2, bm = 32 * tm;
+    const int cap = experts + (batch + bm - 1) / bm;  // sum over experts of ceil(rows / bm)
+    // one launch with 32-bit offsets: each expert's codes below 2^31 bytes, and
+    // the rows of x, which are otherwise gathered first
     if (int64_t(N) * K * t.bits / 8 >= (int64_t(1) << 31) || int64_t(batch) * K * 2 >= (int64_t(1) << 31)) return false;
-    const size_t xg_bytes = (size_t(batch) * size_t(K) * 2u + 255u) & ~size_t(255);
+    const bool direct = x_batches * int64_t(K) * 2 < (int64_t(1) << 31);
+    const size_t xg_bytes = direct ? 0 : (size_t(batch) * size_t(K) * 2u + 255u) & ~size_t(255);
     void* ws = ws_acquire(src, xg_bytes + size_t(cap) * sizeof(int4), st);
     if (!ws) return false;
     uint16_t* xg = reinterpret_cast<uint16_t*>(ws);
     int4* list = reinterpret_cast<int4*>(reinterpret_cast<char*>(ws) + xg_bytes);
     const int64_t yn = int64_t(batch) * N;
-    qmm_zero<<<dim3(unsigned(yn / 1024 < 4096 ? yn / 1024 + 1 : 4096)), dim3(256), 0, st>>>(y, yn);
-    qmm_gather_rows<<<dim3(unsigned(batch)), dim3(256), 0, st>>>(xg, x, lhs, x_batches, K);
-    qmm_group_tiles<<<dim3(1), dim3(1024), 0, st>>>(list, rhs, batch, experts, cap);
+    qmm_group_prepare<<<dim3(1 + unsigned(yn / 4096 < 1024 ? yn / 4096 + 1 : 1024)), dim3(1024), 0, st>>>(
+        list, rhs, batch, experts, cap, bm, y, yn);
+    if (!direct) qmm_gather_rows<<<dim3(unsigned(batch)), dim3(256), 0, st>>>(xg, x, lhs, x_batches, K);
     QmmArgs a{};
-    a.y = y, a.x = xg, a.w = w, a.s = static_cast<const uint16_t*>(s), a.b = static_cast<const uint16_t*>(b);
+    a.y = y, a.x = direct ? x : xg, a.w = w, a.s = static_cast<const uint16_t*>(s), a.b = static_cast<const uint16_t*>(b);
     a.M = batch, a.N = N, a.K = K, a.ldy = N;
-    a.mtiles = cap, a.ntiles = (N + kBN - 1) / kBN, a.splits = 1, a.cps = K / kBK;
+    a.mtiles = cap, a.ntiles = (N + 128 * tn - 1) / (128 * tn), a.splits = 1, a.cps = K / kBK;
     a.groups = list;
-    return qmm_run(4, 2, t, a, a.mtiles * a.ntiles, st);
+    a.lhs = direct ? lhs : nullptr, a.x_rows = direct ? int(x_batches) : batch;
+    return qmm_run(tm, tn, t, a, a.mtiles * a.ntiles, st);
 }
 
 bool launch_qmm_grouped(int bits, int gs, int scale_dtype, uint16_t* y, const uint16_t* x, const uint32_t* w,

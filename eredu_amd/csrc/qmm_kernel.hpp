@@ -143,6 +143,10 @@ struct QmmArgs {
     // weights, scales and biases follow the previous expert's.  An expert
     // below zero marks an unused entry.  Null: one plain problem.
     const int4* groups;
+    // Grouped: y row r multiplies x row lhs[r] (null: row r, or row 0 of a
+    // single one) of x_rows; an index outside them reads zeros.
+    const int32_t* lhs;
+    int x_rows;
 };
 
 // PW (parameter windows, group sizes 32, 64 and 128 with 4-byte aligned rows
@@ -155,9 +159,11 @@ struct QmmArgs {
 // TM x TN: 32-row blocks and 32-column blocks of each wave's output block;
 // the workgroup's tile is 32 TM rows x 128 TN columns (4 x 2: 128 x 256, the
 // default; 4 x 1 and 2 x 1: 128 x 128 and 64 x 128, for outputs with too few
-// large tiles to fill the GPU, which then need no split of K or fewer splits).
+// large tiles to fill the GPU, which then need no split of K or fewer splits;
+// 3 x 1: 96 x 128).  A 2 x 1 workgroup leaves room for a second one on its CU
+// (72 KiB of LDS, 80 registers): routed experts of 32 rows 252 -> 218 us.
 template <int BITS, int GS, typename ST, bool PW, typename XT, int TM, int TN>
-__global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void qmm_mfma_kernel(
+__global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, TM == 2 ? 4 : 2))) void qmm_mfma_kernel(
     const QmmArgs args) {
     constexpr int BM = 32 * TM, BN = 128 * TN, LBUF = BM * kBK * 2;  // LBUF: bytes per K-group buffer
     static_assert((TM == 4 && TN == 2) || (TM >= 2 && TM <= 4 && TN == 1), "tile shapes");
@@ -192,10 +198,11 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const char* sp = reinterpret_cast<const char*>(args.s);
     const char* bp = reinterpret_cast<const char*>(args.b);
     uint16_t* yp = args.y;
+    int first = 0, x_rows = M;
     if (args.groups) {
         const int4 gd = args.groups[tm];
         if (gd.x < 0) return;  // unused entry: the whole workgroup leaves before any barrier
-        xp += int64_t(gd.y) * K;
+        first = gd.y, x_rows = args.x_rows;
         yp += int64_t(gd.y) * args.ldy;
         M = gd.z;
         m0 = gd.w;
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const int steps = (nloc + 1) / 2;         // chunks of the first K-group
     const int mine = (nloc - kgrp + 1) / 2;   // of this one (the second may have one fewer, or none)
 
-    const __amdgpu_buffer_rsrc_t xr = raw_rsrc(xp, uint32_t(M) * uint32_t(K) * 2u);
+    const __amdgpu_buffer_rsrc_t xr = raw_rsrc(xp, uint32_t(x_rows) * uint32_t(K) * 2u);
     const uint32_t row_bytes = uint32_t(K) * BITS / 8u;  // (the launcher keeps N * row_bytes below 2^31)
     const __amdgpu_buffer_rsrc_t wr = raw_rsrc(wp, uint32_t(N) * row_bytes);
     const __amdgpu_buffer_rsrc_t sr = raw_rsrc(sp, uint32_t(N) * uint32_t(G) * PB);
@@ -241,7 +248,14 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         const int row = 8 * (TM * wave + i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
-        a_goff[i] = m0 + row < M ? (uint32_t(m0 + row) * uint32_t(K) + uint32_t(8 * c)) * 2u : kOutOfRange;
+        int src = m0 + row;
+        bool live = src < M;
+        if (args.groups) {
+            // (the routes' rows are read where they are: no gathered copy)
+            if (live) src = args.lhs ? args.lhs[first + src] : x_rows == 1 ? 0 : first + src;
+            live = live && src >= 0 && src < x_rows;
+        }
+        a_goff[i] = live ? (uint32_t(src) * uint32_t(K) + uint32_t(8 * c)) * 2u : kOutOfRange;
     }
     // Codes, too, go straight to LDS: per step a row's 128 codes (its chunks of
     // both K-groups, 16 BITS bytes), load q of wave v = 4 kgrp + wave filling the

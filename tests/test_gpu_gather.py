@@ -283,3 +283,23 @@ def test_grouped_and_per_route_paths_on_a_mixtral_like_layout(cuda):
     for hint in (True, False):
         y = gather_qmm(*args, sorted_indices=hint)
         check(y, y_ref, out_is_bf16=True)
+
+
+@pytest.mark.parametrize("R,E,lhs_kind", [(64, 32, "none"), (768, 8, "picked"), (784, 8, "picked"), (300, 4, "one"),
+                                          (8200, 128, "picked")])
+def test_grouped_tile_choice_and_row_sources(cuda, R, E, lhs_kind):
+    """Means of 2, 96 (the last 64-row tiles), 98 and 75 rows per expert, more
+    routes than the prepare kernel holds in LDS; x rows read in place through
+    lhs (out-of-range ones read zeros), row by row, or one row for all; the
+    first and last routes outside the bank (zero rows)."""
+    from eredu_amd import gather_qmm
+
+    N, K, gs, bits = 128, 128, 64, 4
+    rng = np.random.default_rng(R + E)
+    rhs = np.sort(rng.integers(0, E, R)).astype(np.int32)
+    rhs[:3], rhs[-2:] = -1, E
+    Bx = {"none": R, "picked": 40, "one": 1}[lhs_kind]
+    lhs = np.arange(R) if lhs_kind == "none" else np.zeros(R, np.int64) if lhs_kind == "one" else rng.integers(0, Bx, R)
+    if lhs_kind == "picked":
+        lhs[[5, R // 2]] = [-1, Bx]
+    run(E, N, K, gs, bits, lhs, rhs, Bx=Bx, seed=R, sorted_indices=True)
