@@ -84,6 +84,8 @@ def lib() -> ctypes.CDLL:
     EREDU_AMD_LIB environment variable names (another build of it, e.g. the
     sanitizer build of the host code that tests/test_host_sanitize.py makes)."""
     global _lib
+    if _lib is not None:  # (published complete, below)
+        return _lib
     with _lock:
         if _lib is None:
             path = os.environ.get("EREDU_AMD_LIB") or LIB_PATH

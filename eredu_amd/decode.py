@@ -33,6 +33,7 @@ import torch
 
 from . import _native
 from ._native import check
+from .quantization import _stream
 
 HEAD_DIM = 128
 
@@ -55,10 +56,6 @@ def llama3_rope_freqs(dims: int, base: float, factor: float = 8.0, low_freq_fact
     smooth = ((f32(1.0) / wl) * old - f32(low_freq_factor)) / f32(high_freq_factor - low_freq_factor)
     freqs = np.where(medium, freqs / ((f32(1.0) - smooth) / f32(factor) + smooth), freqs).astype(f32)
     return freqs
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def _bf16(t: torch.Tensor, what: str) -> None:

@@ -18,6 +18,7 @@ import torch
 
 from . import _native
 from ._native import EreduError, check
+from .quantization import _stream
 
 
 class GgmlType(enum.IntEnum):
@@ -238,7 +239,7 @@ def convert_affine(desc: TensorDescriptor, raw: torch.Tensor, endian: Endian = E
     check(
         _native.lib().eq_gguf_convert_affine(
             weights.data_ptr(), scales.data_ptr(), biases.data_ptr(), raw.data_ptr(), raw.numel(),
-            int(ty), rows, cols, int(endian), torch.cuda.current_stream().cuda_stream,
+            int(ty), rows, cols, int(endian), _stream(),
         )
     )
     weight_shape = shape[:-1] + [cols * bits // 32]
@@ -270,7 +271,7 @@ def dequantize(
     check(
         _native.lib().eq_gguf_dequantize(
             out.data_ptr(), raw.contiguous().data_ptr(), raw.numel(), int(ty), rows, cols, int(endian),
-            int(definition), code, torch.cuda.current_stream().cuda_stream,
+            int(definition), code, _stream(),
         )
     )
     return out
@@ -305,7 +306,7 @@ def embedding(
     check(
         _native.lib().eq_gguf_embedding(
             out.data_ptr(), raw.contiguous().data_ptr(), raw.numel(), int(ty), rows, cols, ids.data_ptr(),
-            ids.numel(), int(endian), code, torch.cuda.current_stream().cuda_stream,
+            ids.numel(), int(endian), code, _stream(),
         )
     )
     return out
@@ -345,7 +346,7 @@ def native_grouped_linear(input: torch.Tensor, weight: "NativeTensor", group_ids
         _native.lib().eq_gguf_grouped_linear(
             y.data_ptr(), x.data_ptr(), weight.data.contiguous().data_ptr(), weight.data.numel(), int(ty), experts,
             N, K, ids.data_ptr(), routes, int(weight.endian), _native.EQ_DTYPE_BF16, sorted_ids,
-            torch.cuda.current_stream().cuda_stream,
+            _stream(),
         )
     )
     return y
@@ -372,7 +373,7 @@ def linear(x: torch.Tensor, desc: TensorDescriptor, raw: torch.Tensor, endian: E
     check(
         _native.lib().eq_gguf_linear(
             y.data_ptr(), x2.data_ptr(), raw.contiguous().data_ptr(), raw.numel(), int(ty), x2.shape[0], N, K,
-            int(endian), _native.EQ_DTYPE_BF16, torch.cuda.current_stream().cuda_stream,
+            int(endian), _native.EQ_DTYPE_BF16, _stream(),
         )
     )
     return y.reshape(*x.shape[:-1], N)
@@ -467,7 +468,7 @@ def convert_mxfp4(desc: TensorDescriptor, raw: torch.Tensor) -> MxFp4Tensor:
     check(
         _native.lib().eq_gguf_convert_mxfp4(
             weights.data_ptr(), scales.data_ptr(), raw.contiguous().data_ptr(), raw.numel(), rows, cols,
-            torch.cuda.current_stream().cuda_stream,
+            _stream(),
         )
     )
     weight_shape = shape[:-1] + [cols // 8]

@@ -50,8 +50,29 @@ def quantized_packed_dimension(dimension: int, bits: int) -> int:
     return dimension * bits // 32
 
 
+# The current stream's handle of the current device, without building the
+# torch.cuda.Stream object around it (1.5 us of a call's ~12).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _get_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_get_device())
+
+
+def _rows(x: torch.Tensor, K: int) -> torch.Tensor:
+    """x [..., K] as contiguous rows [M, K] (x itself where it is that)."""
+    if x.dim() == 2 and x.is_contiguous():
+        return x
+    return x.reshape(-1, K).contiguous()
+
+
+_MODE_NAME = {}  # QuantizationMode -> its name in bytes, as the C ABI takes it
+
+
+_MODE_NAME.update({m: m.value.encode() for m in QuantizationMode})
 
 
 def _dtype_code(t: torch.Tensor, what: str) -> int:
@@ -124,7 +145,7 @@ def quantized_matmul_with_mode(
     N, K = _check_operands(x, w, scales, biases, transpose, group_size, bits)
     x_code = _dtype_code(x, "x")
     s_code = _scale_code(scales, mode)
-    x2 = x.reshape(-1, K).contiguous()
+    x2 = _rows(x, K)
     M = x2.shape[0]
     w = w.contiguous()
     scales = scales.contiguous()
@@ -134,10 +155,10 @@ def quantized_matmul_with_mode(
         _native.lib().eq_quantized_matmul(
             y.data_ptr(), x2.data_ptr(), w.data_ptr(), scales.data_ptr(),
             biases.data_ptr() if biases is not None else None,
-            M, N, K, bool(transpose), int(group_size), int(bits), mode.value.encode(), x_code, s_code, _stream(),
+            M, N, K, bool(transpose), int(group_size), int(bits), _MODE_NAME[mode], x_code, s_code, _stream(),
         )
     )
-    return y.reshape(*x.shape[:-1], N)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
 
 
 def quantized_matmul(
@@ -175,9 +196,9 @@ def _check_operands(x, w, scales, biases, transpose, group_size, bits):
     if group_size <= 0 or packed_dim % group_size != 0:
         raise EreduError(f"the quantized dimension {packed_dim} is not divisible by group_size {group_size}")
     expect_scales = (w.shape[0], packed_dim // group_size)
-    if tuple(scales.shape) != expect_scales:
+    if scales.shape != expect_scales:
         raise EreduError(f"scales has shape {tuple(scales.shape)}, expected {expect_scales}")
-    if biases is not None and (tuple(biases.shape) != expect_scales or biases.dtype != scales.dtype):
+    if biases is not None and (biases.shape != expect_scales or biases.dtype != scales.dtype):
         raise EreduError("biases must match scales in shape and dtype")
     return N, K
 
@@ -208,7 +229,7 @@ def quantized_matmul_batched(
         N, K = _check_operands(x, w, scales, biases, transpose, group_size, bits)
         if x.dtype != x0.dtype or scales.dtype != s0.dtype:
             raise EreduError("all problems of a batch must share the activation and scale dtypes")
-        x2 = x.reshape(-1, K).contiguous()
+        x2 = _rows(x, K)
         if M is None:
             M = x2.shape[0]
         elif x2.shape[0] != M:
@@ -222,11 +243,32 @@ def quantized_matmul_batched(
                                     biases.data_ptr() if biases is not None else None, N, K)
     check(
         _native.lib().eq_quantized_matmul_batched(
-            arr, len(problems), M, bool(transpose), int(group_size), int(bits), mode.value.encode(), x_code, s_code,
+            arr, len(problems), M, bool(transpose), int(group_size), int(bits), _MODE_NAME[mode], x_code, s_code,
             _stream(),
         )
     )
-    return [y.reshape(*lead, N) for y, lead, N in outs]
+    return [y if len(lead) == 1 else y.reshape(*lead, N) for y, lead, N in outs]
+
+
+def _broadcast_indices(lhs_indices, rhs_indices, x_batches, w_batches, xb_shape, wb_shape, dev):
+    """(output batch shape, flat int32 lhs, flat int32 rhs) by MLX's rules:
+    an absent array is arange over its operand's batch shape, and the two
+    broadcast to the output batch shape."""
+    if lhs_indices is None:
+        lhs_indices = torch.arange(x_batches, device=dev, dtype=torch.int32).reshape(xb_shape)
+    if rhs_indices is None:
+        rhs_indices = torch.arange(w_batches, device=dev, dtype=torch.int32).reshape(wb_shape)
+    for name, idx in (("lhs_indices", lhs_indices), ("rhs_indices", rhs_indices)):
+        if idx.dtype.is_floating_point or idx.dtype.is_complex or idx.dtype == torch.bool:
+            raise EreduError(f"{name} must be an integer array, got {idx.dtype}")
+    try:
+        batch_shape = torch.broadcast_shapes(lhs_indices.shape, rhs_indices.shape)
+    except RuntimeError as e:
+        raise EreduError(f"lhs_indices {tuple(lhs_indices.shape)} and rhs_indices "
+                         f"{tuple(rhs_indices.shape)} do not broadcast") from e
+    lhs = lhs_indices.to(torch.int32).broadcast_to(batch_shape).contiguous().reshape(-1)
+    rhs = rhs_indices.to(torch.int32).broadcast_to(batch_shape).contiguous().reshape(-1)
+    return batch_shape, lhs, rhs
 
 
 def gather_qmm_with_mode(
@@ -277,21 +319,18 @@ def gather_qmm_with_mode(
     N, K = _check_operands(x, w2[0], s2[0], b2[0] if b2 is not None else None, transpose, group_size, bits)
     M = x.shape[-2]
     dev = x.device
-    if lhs_indices is None:
-        lhs_indices = torch.arange(x_batches, device=dev, dtype=torch.int32).reshape(xb_shape)
-    if rhs_indices is None:
-        rhs_indices = torch.arange(w_batches, device=dev, dtype=torch.int32).reshape(wb_shape)
-    for name, idx in (("lhs_indices", lhs_indices), ("rhs_indices", rhs_indices)):
-        if idx.dtype.is_floating_point or idx.dtype.is_complex or idx.dtype == torch.bool:
-            raise EreduError(f"{name} must be an integer array, got {idx.dtype}")
-    try:
-        batch_shape = torch.broadcast_shapes(lhs_indices.shape, rhs_indices.shape)
-    except RuntimeError as e:
-        raise EreduError(f"lhs_indices {tuple(lhs_indices.shape)} and rhs_indices "
-                         f"{tuple(rhs_indices.shape)} do not broadcast") from e
-    lhs = lhs_indices.to(torch.int32).broadcast_to(batch_shape).contiguous().reshape(-1)
-    rhs = rhs_indices.to(torch.int32).broadcast_to(batch_shape).contiguous().reshape(-1)
-    batch = lhs.numel()
+    # the common routed calls: flat int32 indices, one per x row or with x rows
+    # in order (which the C ABI takes as no lhs at all)
+    flat = (rhs_indices is not None and rhs_indices.dtype == torch.int32 and rhs_indices.dim() == 1 and
+            rhs_indices.is_contiguous())
+    if flat and lhs_indices is None and tuple(rhs_indices.shape) == xb_shape:
+        batch_shape, lhs, rhs = xb_shape, None, rhs_indices
+    elif (flat and lhs_indices is not None and lhs_indices.dtype == torch.int32 and lhs_indices.is_contiguous() and
+          lhs_indices.shape == rhs_indices.shape):
+        batch_shape, lhs, rhs = tuple(rhs_indices.shape), lhs_indices, rhs_indices
+    else:
+        batch_shape, lhs, rhs = _broadcast_indices(lhs_indices, rhs_indices, x_batches, w_batches, xb_shape, wb_shape, dev)
+    batch = rhs.numel()
     x3 = x.reshape(x_batches, M, K).contiguous()
     w2, s2 = w2.contiguous(), s2.contiguous()
     b2 = b2.contiguous() if b2 is not None else None
@@ -299,8 +338,8 @@ def gather_qmm_with_mode(
     check(
         _native.lib().eq_gather_qmm(
             y.data_ptr(), x3.data_ptr(), w2.data_ptr(), s2.data_ptr(), b2.data_ptr() if b2 is not None else None,
-            lhs.data_ptr(), rhs.data_ptr(), batch, x_batches, w_batches, M, N, K, bool(transpose),
-            int(group_size), int(bits), mode.value.encode(), _dtype_code(x, "x"), _scale_code(scales, mode),
+            lhs.data_ptr() if lhs is not None else None, rhs.data_ptr(), batch, x_batches, w_batches, M, N, K,
+            bool(transpose), int(group_size), int(bits), _MODE_NAME[mode], _dtype_code(x, "x"), _scale_code(scales, mode),
             bool(sorted_indices), _stream(),
         )
     )

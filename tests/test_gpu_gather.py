@@ -303,3 +303,29 @@ def test_grouped_tile_choice_and_row_sources(cuda, R, E, lhs_kind):
     if lhs_kind == "picked":
         lhs[[5, R // 2]] = [-1, Bx]
     run(E, N, K, gs, bits, lhs, rhs, Bx=Bx, seed=R, sorted_indices=True)
+
+
+@pytest.mark.parametrize("form", ["int64", "strided", "column", "lhs given", "one row"])
+def test_index_forms_agree_with_the_flat_int32_call(cuda, form):
+    """Flat int32 indices go to the C ABI as they are (absent lhs as none); the
+    other forms through the broadcast rules: bit-equal results."""
+    from eredu_amd import gather_qmm
+
+    R, E, N, K = 6, 4, 256, 512
+    w, s, b = expert_bank(E, N, K, 64, 4, orc.BF16, 3)
+    _, xd = activations(1 if form == "one row" else R, 1, K, orc.BF16, 4)
+    args = (dev_words(w), dev_bf16(s), dev_bf16(b))
+    rhs = torch.tensor([3, 0, 1, 1, 2, 0], dtype=torch.int32, device="cuda")
+    rows = torch.zeros(R, dtype=torch.int32, device="cuda") if form == "one row" else \
+        torch.arange(R, dtype=torch.int32, device="cuda")
+    flat = gather_qmm(xd, *args, rows, rhs)
+    if form == "int64":
+        other = gather_qmm(xd, *args, None, rhs.long())
+    elif form == "strided":
+        other = gather_qmm(xd, *args, None, torch.stack([rhs, rhs], 1)[:, 0])
+    elif form == "column":
+        other = gather_qmm(xd.reshape(R, 1, 1, K), *args, None, rhs.reshape(R, 1)).reshape(R, 1, N)
+    else:
+        other = gather_qmm(xd, *args, None, rhs)
+    assert tuple(other.shape) == (R, 1, N)
+    assert torch.equal(flat, other)
