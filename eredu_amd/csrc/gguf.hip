@@ -390,13 +390,28 @@ __device__ __forceinline__ uint32_t lds_half(const uint8_t* b, int o) {
     return BIG ? (uint32_t(b[o]) << 8) | b[o + 1] : uint32_t(b[o]) | (uint32_t(b[o + 1]) << 8);
 }
 
-// 8 bytes at an even LDS offset as two words: byte j in byte j % 4 of lo (j < 4)
-// or hi.  Blocks of 22 / 110 / 210 bytes sit at 2-byte alignment in LDS, so
-// the words are assembled from 16-bit reads.
+// 8 bytes at an LDS offset of a block of type T as two words: byte j in byte
+// j % 4 of lo (j < 4) or hi.  Blocks of 18 / 22 / 110 / 210 bytes sit at 2-byte
+// alignment in LDS, where the compiler would merge the reads into wide
+// unaligned ones, which the LDS serves with many stalls (Q6_K linear, 128256 x
+// 4096, M = 1: 62 of 74 M busy LDS cycles were such stalls): there the words
+// around the bytes are read aligned and shifted (that call 161 -> 141 us,
+// 4096 x 14336 23.9 -> 20.9, the Q6_K prefill's re-pack with its product at M =
+// 512, 4096 x 4096, 58.5 -> 50.7 with the product's own change).  The third of
+// them is read only when the bytes reach into it.
+template <int T, bool ALIGNED>
 __device__ __forceinline__ void lds_8b(const uint8_t* p, uint32_t& lo, uint32_t& hi) {
-    const uint16_t* q = reinterpret_cast<const uint16_t*>(p);
-    lo = uint32_t(q[0]) | (uint32_t(q[1]) << 16);
-    hi = uint32_t(q[2]) | (uint32_t(q[3]) << 16);
+    if constexpr (KQuant<T>::bytes % 4 == 0 || !ALIGNED) {
+        const uint16_t* q = reinterpret_cast<const uint16_t*>(p);
+        lo = uint32_t(q[0]) | (uint32_t(q[1]) << 16);
+        hi = uint32_t(q[2]) | (uint32_t(q[3]) << 16);
+    } else {
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(__builtin_align_down(p, 4));
+        const uint32_t odd = (uint32_t(reinterpret_cast<uintptr_t>(p)) >> 1) & 1u;
+        const uint32_t w0 = q[0], w1 = q[1], w2 = q[1 + odd];
+        lo = __builtin_amdgcn_alignbit(w1, w0, 16 * odd);
+        hi = __builtin_amdgcn_alignbit(w2, w1, 16 * odd);
+    }
 }
 
 // Bits 0..3 of t moved to bit 0 of bytes 0..3 (the four shifted copies of t
@@ -406,19 +421,19 @@ __device__ __forceinline__ uint32_t spread4(uint32_t t) { return ((t & 15u) * 0x
 // Codes of values i0 .. i0 + 7 (i0 a multiple of 8) of unit u of a block, as
 // byte lanes: value i0 + j in byte j % 4 of c0 (j < 4) or c1.  Every code of
 // a byte lane is extracted by one shift and mask of the word.
-template <int T, bool BIG>
+template <int T, bool BIG, bool ALIGNED = true>
 __device__ __forceinline__ void kq_codes8(const uint8_t* b, int u, int i0, uint32_t& c0, uint32_t& c1) {
     uint32_t a0, a1, h0, h1;
     if constexpr (T == EQ_GGML_IQ4_NL || T == EQ_GGML_IQ4_XS) {
         // level indices: byte 2 + i (IQ4_NL) or 8 + 16 ib + i (IQ4_XS, unit = group ib)
         // holds value i in its low nibble and value 16 + i in its high (iquant.rs:271-301)
-        lds_8b(b + (T == EQ_GGML_IQ4_NL ? 2 : 8 + 16 * u) + (i0 & 15), a0, a1);
+        lds_8b<T, ALIGNED>(b + (T == EQ_GGML_IQ4_NL ? 2 : 8 + 16 * u) + (i0 & 15), a0, a1);
         const int sh = (i0 >> 4) * 4;
         c0 = (a0 >> sh) & 0x0f0f0f0fu;
         c1 = (a1 >> sh) & 0x0f0f0f0fu;
     } else if constexpr (T == EQ_GGML_Q4_1) {
         // low nibbles of bytes 4..20 are values 0..15, high nibbles 16..31 (convert.rs:367-370)
-        lds_8b(b + 4 + (i0 & 15), a0, a1);
+        lds_8b<T, ALIGNED>(b + 4 + (i0 & 15), a0, a1);
         const int sh = (i0 >> 4) * 4;
         c0 = (a0 >> sh) & 0x0f0f0f0fu;
         c1 = (a1 >> sh) & 0x0f0f0f0fu;
@@ -426,7 +441,7 @@ __device__ __forceinline__ void kq_codes8(const uint8_t* b, int u, int i0, uint3
         // nibbles as Q4_1 at 6 / 8, plus bit i of the u32 at 2 / 4 as bit 4 (convert.rs:553-562):
         // bits i0 .. i0 + 7 are byte i0 / 8 of that word in its byte order
         constexpr int qh = T == EQ_GGML_Q5_0 ? 2 : 4, qs = qh + 4;
-        lds_8b(b + qs + (i0 & 15), a0, a1);
+        lds_8b<T, ALIGNED>(b + qs + (i0 & 15), a0, a1);
         const int sh = (i0 >> 4) * 4;
         const uint32_t hb = b[qh + (BIG ? 3 - (i0 >> 3) : (i0 >> 3))];
         c0 = ((a0 >> sh) & 0x0f0f0f0fu) | (spread4(hb) << 4);
@@ -434,23 +449,23 @@ __device__ __forceinline__ void kq_codes8(const uint8_t* b, int u, int i0, uint3
     } else if constexpr (T == EQ_GGML_Q2_K) {
         // group g = 2u + i/16 takes 2 bits at shift 2 ((g % 8) / 2) = 2 (u % 4) of byte
         // 16 + (g / 8) 32 + (g % 2) 16 + i % 16 = 16 + (u / 4) 32 + i (convert.rs:501-505)
-        lds_8b(b + 16 + (u >> 2) * 32 + i0, a0, a1);
+        lds_8b<T, ALIGNED>(b + 16 + (u >> 2) * 32 + i0, a0, a1);
         const int sh = (u & 3) * 2;
         c0 = (a0 >> sh) & 0x03030303u;
         c1 = (a1 >> sh) & 0x03030303u;
     } else if constexpr (T == EQ_GGML_Q3_K) {
         // as Q2_K at byte 32, plus bit g / 2 = u of hm[(g % 2) 16 + i % 16] = hm[i] as bit 2
         // (convert.rs:531-539)
-        lds_8b(b + 32 + (u >> 2) * 32 + i0, a0, a1);
-        lds_8b(b + i0, h0, h1);
+        lds_8b<T, ALIGNED>(b + 32 + (u >> 2) * 32 + i0, a0, a1);
+        lds_8b<T, ALIGNED>(b + i0, h0, h1);
         const int sh = (u & 3) * 2;
         c0 = ((a0 >> sh) & 0x03030303u) | (((h0 >> u) & 0x01010101u) << 2);
         c1 = ((a1 >> sh) & 0x03030303u) | (((h1 >> u) & 0x01010101u) << 2);
     } else if constexpr (T == EQ_GGML_Q5_K) {
         // unit = group g: nibble g % 2 of qs[(g / 2) 32 + i] at 48, bit g of qh[i] at 16
         // as bit 4 (convert.rs:453-461)
-        lds_8b(b + 48 + (u >> 1) * 32 + i0, a0, a1);
-        lds_8b(b + 16 + i0, h0, h1);
+        lds_8b<T, ALIGNED>(b + 48 + (u >> 1) * 32 + i0, a0, a1);
+        lds_8b<T, ALIGNED>(b + 16 + i0, h0, h1);
         const int sh = (u & 1) * 4;
         c0 = ((a0 >> sh) & 0x0f0f0f0fu) | (((h0 >> u) & 0x01010101u) << 4);
         c1 = ((a1 >> sh) & 0x0f0f0f0fu) | (((h1 >> u) & 0x01010101u) << 4);
@@ -459,8 +474,8 @@ __device__ __forceinline__ void kq_codes8(const uint8_t* b, int u, int i0, uint3
         // ql[h 64 + (k % 2) 32 + i], bits 2k, 2k + 1 of qh[128 + h 32 + i] as bits 4, 5
         // (convert.rs:472-477)
         const int h = u >> 2, k = u & 3;
-        lds_8b(b + h * 64 + (k & 1) * 32 + i0, a0, a1);
-        lds_8b(b + 128 + h * 32 + i0, h0, h1);
+        lds_8b<T, ALIGNED>(b + h * 64 + (k & 1) * 32 + i0, a0, a1);
+        lds_8b<T, ALIGNED>(b + 128 + h * 32 + i0, h0, h1);
         const int sh = (k >> 1) * 4;
         c0 = ((a0 >> sh) & 0x0f0f0f0fu) | (((h0 >> (2 * k)) & 0x03030303u) << 4);
         c1 = ((a1 >> sh) & 0x0f0f0f0fu) | (((h1 >> (2 * k)) & 0x03030303u) << 4);
@@ -906,13 +921,21 @@ __global__ __launch_bounds__(256) void q4k_linear(uint16_t* __restrict__ y, cons
 // sum x q = e - 128 sum x.  Up to kLinRows activation rows per launch.
 
 constexpr int kKqStageVec = 8;  // 16-byte pieces per lane of one staged row group
+constexpr int64_t kKqXLds = 40 * 1024;  // LDS per workgroup up to which x is staged as well
 
 // Persistent workgroups walk row groups grp, grp + gridDim.x, ...; a full
 // group on a 16-byte-aligned payload is fetched into registers one group
 // ahead (its loads in flight while the current group is multiplied), a
 // ragged or unaligned one is staged with 2-byte loads when its turn comes.
 // Sums of x over every group of K are taken once per launch into LDS.
-template <int T, bool BIG, bool MANY, int W>
+//
+// XL: x is staged in LDS too, 16-byte piece j of unit u at [j][u], so that the
+// 64 lanes of a unit step read consecutive pieces.  From memory the same reads
+// are 64 bytes apart, a cache line per two lanes, and every weight row costs
+// 256 cycles of the texture unit per 64 units: with the codes read aligned
+// that unit was busy for 93 % of the launch.  M = 1 at K = 4096: Q6_K 14336 rows
+// 19.9 -> 18.8 us, 128256 rows 141 -> 136, Q5_K 32768 rows 34.7 -> 32.0.
+template <int T, bool BIG, bool MANY, int W, bool XL>
 __global__ __launch_bounds__(64 * W) void kq_linear(uint16_t* __restrict__ y, const uint16_t* __restrict__ x,
                                                     const uint8_t* __restrict__ raw, int M, int N, int K, int R,
                                                     bool vec_ok, ExpertSel sel) {
@@ -942,6 +965,14 @@ __global__ __launch_bounds__(64 * W) void kq_linear(uint16_t* __restrict__ y, co
             sx = dot2_bf16(v.w, kBf16Ones, sx);
         }
         sxs[i] = sx;
+    }
+    uint4* xl = reinterpret_cast<uint4*>(reinterpret_cast<uint8_t*>(sxs) + ((M * ngk * 4 + 15) & ~15));
+    if constexpr (XL) {
+        const uint4* xp = reinterpret_cast<const uint4*>(x);
+        for (int i = threadIdx.x; i < M * 4 * U; i += NT) {
+            const int m = i / (4 * U), c = i - m * 4 * U;
+            xl[(m * 4 + (c & 3)) * U + (c >> 2)] = xp[i];
+        }
     }
     const int64_t ngroups = (int64_t(N) + R - 1) / R;
     auto pipelined = [&](int64_t gi) { return vec_ok && (gi + 1) * R <= N; };
@@ -987,7 +1018,9 @@ __global__ __launch_bounds__(64 * W) void kq_linear(uint16_t* __restrict__ y, co
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     uint32_t c0, c1;
-                    kq_codes8<T, BIG>(b, uu, 8 * q, c0, c1);
+                    // (with several activation rows the x reads set the time, and the
+                    // shifts only add to it: 4096 x 14336, M = 8, 79.0 against 81.9 us)
+                    kq_codes8<T, BIG, !MANY>(b, uu, 8 * q, c0, c1);
                     if constexpr (P::levels) {
                         // level + 128 (up to 241: exact in bf16, past the 0x43 trick's
                         // range) converted per byte
@@ -1013,7 +1046,7 @@ __global__ __launch_bounds__(64 * W) void kq_linear(uint16_t* __restrict__ y, co
                     uint32_t xw[16];
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const uint4 v = xp[i];
+                        const uint4 v = XL ? xl[(m * 4 + i) * U + u] : xp[i];
                         xw[4 * i] = v.x, xw[4 * i + 1] = v.y, xw[4 * i + 2] = v.z, xw[4 * i + 3] = v.w;
                     }
 #pragma unroll
@@ -1922,7 +1955,12 @@ int native_linear_run(void* y, const void* x, const uint8_t* raw, int ggml_type,
                     constexpr bool B = decltype(b)::value;
                     for (int64_t m0 = 0; m0 < M; m0 += mcap) {
                         const int mc = int(M - m0 < mcap ? M - m0 : mcap);
-                        const int lds = int(rows_lds + mc * sx_row);
+                        // x in LDS for one activation row, while the four workgroups of a CU
+                        // still fit (K = 14336: 20.9 -> 26.6 us with fewer) and walk more than
+                        // one group each (1024 x 4096: 6.2 -> 6.4)
+                        const int64_t with_x = rows_lds + (mc * sx_row + 15) / 16 * 16 + int64_t(mc) * K * 2;
+                        const bool xl = mc == 1 && with_x <= kKqXLds && groups > cap;
+                        const int lds = int(xl ? with_x : rows_lds + mc * sx_row);
                         auto go = [&](auto kernel) {
                             if (lds > 65536)
                                 (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1932,10 +1970,9 @@ int native_linear_run(void* y, const void* x, const uint8_t* raw, int ggml_type,
                                                                   static_cast<const uint16_t*>(x) + m0 * K, raw, mc,
                                                                   int(N), int(K), R, vec_ok, sel);
                         };
-                        if (mc == 1)
-                            go(kq_linear<T, B, false, W>);
-                        else
-                            go(kq_linear<T, B, true, W>);
+                        if (xl) go(kq_linear<T, B, false, W, true>);
+                        else if (mc == 1) go(kq_linear<T, B, false, W, false>);
+                        else go(kq_linear<T, B, true, W, false>);
                     }
                 }
             }))

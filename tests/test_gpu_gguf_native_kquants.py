@@ -79,6 +79,16 @@ def test_native_linear_big_endian_and_unaligned_payload(cuda, ty):
     run_case(ty, 200, 2048, 1, seed=8, offset=2)
 
 
+# One activation row staged in LDS beside the rows: more than four row groups
+# per CU (8 rows each), the last one partial; odd and even superblock counts
+# (Q6_K rows then start at 2-byte and 4-byte offsets); both byte orders.
+@pytest.mark.parametrize("ty", [T.Q5_1, T.Q5K, T.Q6K])
+@pytest.mark.parametrize("K,endian", [(256, G.Endian.Little), (1280, G.Endian.Big), (2048, G.Endian.Little)])
+def test_native_linear_staged_row(cuda, ty, K, endian):
+    print(f"[case] native {ty.name} N=8205 K={K} M=1 {endian!r}", flush=True)
+    run_case(ty, 8205, K, 1, seed=K + int(ty), endian=endian)
+
+
 def test_native_q6k_row_longer_than_64k(cuda):
     """One Q6_K row of 400 superblocks (84000 bytes): one row per workgroup
     with LDS raised past 64 KB."""
