@@ -74,15 +74,24 @@ static int qmm_splits(int tiles, int slots, int nchunks) {
 // its steps of two chunks in `step` each (64, 96 and 128 rows measured at
 // 0.70, 0.87 and 1.0 us, whether or not a second workgroup shares the CU)
 // after 5 us of launch, first loads and reduction; partials are written and
-// read back at 4 MB/us, and their reduction is a launch of 2.5 us.
+// read back at 4 MB/us, and their reduction is a launch of 2.5 us.  Where the
+// 64 x 128 tiles cover more than half the CUs and K is short, K is split only if
+// the pieces stay at 24 chunks, fill 3/4 of the CUs and write partials of at
+// most twice the weight bytes: such calls otherwise need no workspace, and may
+// be captured without an eager call before.
 static QmmPlan qmm_plan_few_rows(int M, int N, int cu, int nchunks, bool may_split) {
     QmmPlan best{};
     double least = 0;
+    const bool short_k = qmm_splits((M + 63) / 64 * ((N + 127) / 128), cu, nchunks) == 1 &&
+                         nchunks / qmm_splits((N + 255) / 256, cu, nchunks) < 32;
     const double step[3] = {0.70, 0.87, 1.0};
     for (int tm = 2; tm <= 4; tm++) {
         const int mt = (M + 32 * tm - 1) / (32 * tm), nt = (N + 127) / 128;
         const int most = may_split ? qmm_splits(mt * nt, cu, nchunks) : 1;
         for (int s = 1; s <= most; s++) {
+            if (s > 1 && short_k &&
+                (nchunks / s < 24 || 4 * mt * nt * s < 3 * cu || int64_t(s) * M * 4 > int64_t(nchunks) * kBK))
+                continue;
             const int rounds = (mt * nt * s + cu - 1) / cu, steps = (nchunks + 2 * s - 1) / (2 * s);
             const double us = rounds * (5.0 + steps * step[tm - 2]) + (s > 1 ? 2.5 + 8.0 * s * M * N / 4e6 : 0.0);
             if (!best.tm || us < least) least = us, best = QmmPlan{tm, 1, mt, nt, s};
