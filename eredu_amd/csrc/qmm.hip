@@ -4,6 +4,7 @@
 #include <mutex>
 
 #include "qmm_kernel.hpp"
+#include "qmm_plan.hpp"
 
 namespace eq {
 
@@ -126,12 +127,6 @@ static QmmPlan qmm_plan(int M, int N, int K, int gs, int bits, bool may_split) {
     return p;
 }
 
-// Parameter windows need whole words: rows of an even number of groups (always
-// so below group size 64) and splits that start at an even group.
-static bool qmm_pw_ok(int gs, int K, int cps) {
-    return gs == 32 || (gs == 64 && (K / 64) % 2 == 0 && cps % 2 == 0) || (gs == 128 && (K / 128) % 2 == 0 && cps % 4 == 0);
-}
-
 // The types of a launch: code bits, group size, scale (EQ_DTYPE_U8: MXFP4) and activation types.
 struct QmmTypes {
     int bits, gs, scale_dtype, x_dtype;
@@ -139,7 +134,7 @@ struct QmmTypes {
 };
 
 static bool qmm_run(int tm, int tn, const QmmTypes& t, const QmmArgs& a, int workgroups, hipStream_t st) {
-    const bool pw = qmm_pw_ok(t.gs, a.K, a.cps);
+    const bool pw = qmm_param_words(t.gs, a.K, a.cps, a.s, a.b);
     if (tn == 2) return qmm_run_t42(t.bits, t.gs, t.scale_dtype, t.x_dtype, pw, a, workgroups, st);
     if (tm == 2) return qmm_run_t21(t.bits, t.gs, t.scale_dtype, t.x_dtype, pw, a, workgroups, st);
     if (tm == 3) return qmm_run_t31(t.bits, t.gs, t.scale_dtype, t.x_dtype, pw, a, workgroups, st);

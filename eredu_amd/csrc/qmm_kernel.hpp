@@ -72,8 +72,6 @@ constexpr int kQmmThreads = 512;               // two K-groups of 4 waves
 // Steps of codes a kernel variant holds in LDS ahead of their use, which is
 // also its main loop's unroll and its parameter windows' length.
 constexpr int qmm_ring(int bits, int tn) { return tn == 2 && bits == 8 ? 2 : 4; }
-// Whether a group size has parameter windows.
-constexpr bool qmm_windows(int gs) { return gs == 32 || gs == 64 || gs == 128; }
 
 typedef _Float16 q_f16x8 __attribute__((ext_vector_type(8)));
 
@@ -149,12 +147,14 @@ struct QmmArgs {
     int x_rows;
 };
 
-// PW (parameter windows, group sizes 32, 64 and 128 with 4-byte aligned rows
-// of scales): instead of a 2-byte load per parameter, column and step, which
-// touches one cache line per row each, the workgroup stages the scales and
-// biases of a window of U steps of both K-groups for all of its columns in
-// LDS: one lane per (array, column, 16 bytes), stored word-major so that a
-// lane reads its column's word of a step without bank conflicts.
+// PW (parameters as whole words: every row of scales and biases 4-byte
+// aligned; otherwise each is a 2-byte load).  Group size 16: the two groups of
+// a lane's codes in one load.  Group sizes 32, 64 and 128 (WIN): windows --
+// instead of a load per parameter, column and step, which touches one cache
+// line per row each, the workgroup stages the scales and biases of a window of
+// U steps of both K-groups for all of its columns in LDS: one lane per (array,
+// column, 16 bytes), stored word-major so that a lane reads its column's word
+// of a step without bank conflicts.
 //
 // TM x TN: 32-row blocks and 32-column blocks of each wave's output block;
 // the workgroup's tile is 32 TM rows x 128 TN columns (4 x 2: 128 x 256, the
@@ -180,7 +180,9 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     constexpr uint32_t PB = MX ? 1u : 2u;  // bytes per scale / bias
     static_assert(!MX || (BITS == 4 && GS == 32 && !PW), "MXFP4: 4-bit codes, group 32");
     static_assert(!MX || std::is_same<XT, BF16T>::value, "MXFP4 prefill takes bf16 activations");
-    static_assert(!PW || GS == 32 || GS == 64 || GS == 128, "parameter windows");
+    static_assert(GS == 16 || GS == 32 || GS == 64 || GS == 128, "group sizes");
+    constexpr bool WIN = PW && GS != 16;
+    constexpr int NPL = GS == 16 && !PW ? 2 : 1;  // loads per parameter, column and step (without windows)
     const int N = args.N, K = args.K, G = K / GS;
     int M = args.M;
 
@@ -230,11 +232,11 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const __amdgpu_buffer_rsrc_t br = raw_rsrc(bp ? bp : sp, bp ? uint32_t(N) * uint32_t(G) * PB : 0u);
     // Parameter windows in LDS: [buffer][scale, bias][word][column]; a word is
     // two consecutive groups (the first in the low half).
-    constexpr int PWW = !PW ? 1 : GS == 32 ? 2 * U : GS == 64 ? U : U / 2;  // words per column and window
+    constexpr int PWW = !WIN ? 1 : GS == 32 ? 2 * U : GS == 64 ? U : U / 2;  // words per column and window
     constexpr int PPR = PWW > 4 ? 2 : 1, PWD = PWW / PPR;                  // pieces per column, words per piece
     constexpr int PIT = (BN * 2 * PPR + kQmmThreads - 1) / kQmmThreads;     // pieces per lane
-    static_assert(!PW || PWW % PPR == 0, "whole pieces");
-    __shared__ uint32_t pbuf[PW ? 2 : 1][2][PWW][PW ? BN : 1];
+    static_assert(!WIN || PWW % PPR == 0, "whole pieces");
+    __shared__ uint32_t pbuf[WIN ? 2 : 1][2][PWW][WIN ? BN : 1];
 
     // Lane offsets (chunk 0); rows past M and columns past N read zero.
     // Activations go straight from memory to LDS: load i of wave w fills the
@@ -312,22 +314,25 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     };
     // One step's parameters of this lane, without windows.
     struct PSlot {
-        uint32_t s[TN], b[TN];
+        uint32_t s[TN][NPL], b[TN][NPL];
     };
     auto load_p = [&](PSlot& S, int i) __attribute__((always_inline)) {
         const uint32_t kp = __builtin_amdgcn_readfirstlane(uint32_t(chunk_k0(i) / GS) * PB);
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             if constexpr (MX) {
-                S.s[j] = __builtin_amdgcn_raw_buffer_load_b8(sr, soff[j], kp, 0);
-                S.b[j] = 0u;
-            } else if constexpr (GS == 16) {
+                S.s[j][0] = __builtin_amdgcn_raw_buffer_load_b8(sr, soff[j], kp, 0);
+                S.b[j][0] = 0u;
+            } else if constexpr (GS == 16 && PW) {
                 // the lane's 32 codes span two groups: both parameters in one word
-                S.s[j] = __builtin_amdgcn_raw_buffer_load_b32(sr, soff[j], kp, 0);
-                S.b[j] = __builtin_amdgcn_raw_buffer_load_b32(br, soff[j], kp, 0);
+                S.s[j][0] = __builtin_amdgcn_raw_buffer_load_b32(sr, soff[j], kp, 0);
+                S.b[j][0] = __builtin_amdgcn_raw_buffer_load_b32(br, soff[j], kp, 0);
             } else {
-                S.s[j] = __builtin_amdgcn_raw_buffer_load_b16(sr, soff[j], kp, 0);
-                S.b[j] = __builtin_amdgcn_raw_buffer_load_b16(br, soff[j], kp, 0);
+#pragma unroll
+                for (int q = 0; q < NPL; q++) {
+                    S.s[j][q] = __builtin_amdgcn_raw_buffer_load_b16(sr, soff[j] + 2 * q, kp, 0);
+                    S.b[j][q] = __builtin_amdgcn_raw_buffer_load_b16(br, soff[j] + 2 * q, kp, 0);
+                }
             }
         }
     };
@@ -410,20 +415,21 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
                            __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            if constexpr (PW) {
+            if constexpr (WIN) {
                 const int col = 32 * TN * wave + 32 * j + l32;
                 // group 32: the chunk's two groups are one word; 64: the groups
                 // of the step's two chunks; 128: those of two steps
                 const int w = GS == 32 ? 2 * r + kgrp : GS == 64 ? r : r / 2;
                 sw[j] = pbuf[buf][0][w][col], bw[j] = pbuf[buf][1][w][col];
             } else {
-                sw[j] = S.s[j], bw[j] = S.b[j];
+                sw[j] = S.s[j][0], bw[j] = S.b[j][0];
+                if constexpr (NPL == 2) sw[j] |= S.s[j][1] << 16, bw[j] |= S.b[j][1] << 16;
             }
         }
     };
     auto params = [&](int r, const uint32_t (&sw)[TN], const uint32_t (&bw)[TN], float (&s)[TN][NG],
                       float (&b)[TN][NG]) __attribute__((always_inline)) {
-        const int sh = !PW ? 0 : GS == 32 ? 16 * kb : GS == 64 ? 16 * kgrp : 16 * (r & 1);
+        const int sh = !WIN ? 0 : GS == 32 ? 16 * kb : GS == 64 ? 16 * kgrp : 16 * (r & 1);
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             if constexpr (MX) {
@@ -482,7 +488,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
         }
     };
 
-    PSlot pring[PW ? 1 : U];
+    PSlot pring[WIN ? 1 : U];
     uint32_t sw[TN], bw[TN];                    // the next chunk's parameter words
     float ps[TN][NG], pb[TN][NG];               // parameters of the chunk being dequantized
     q_u32x4 bq[2][TN];                          // B operands of the current and the next k-step
@@ -496,7 +502,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     // Prologue: the first parameter window, the codes of steps 0 .. U - 1 and
     // the activations of steps 0 and 1 requested; the window stored to LDS,
     // step 0's loads awaited, its first operands prepared.
-    if constexpr (PW) load_pw(0);
+    if constexpr (WIN) load_pw(0);
     else
 #pragma unroll
         for (int c = 0; c < U; c++) load_p(pring[c], c);
@@ -514,7 +520,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     for (int c = 1; c < U; c++)
 #pragma unroll
         for (int q = 0; q < CL; q++) load_c(cbuf(c), c_koff(c), q);
-    if constexpr (PW) store_pw(0);
+    if constexpr (WIN) store_pw(0);
     __builtin_amdgcn_sched_barrier(0);
     wait_lds_and_vmcnt<TM + (U - 1) * CL>();
     barrier();
@@ -542,7 +548,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
                         // are free; the next step's have landed.
                         // (memory operations complete in order, and the newest CL are the
                         // codes requested in the last step, which U = 4 leaves in flight)
-                        if constexpr (PW && r == U - 1) store_pw(pw_cur ^ 1);
+                        if constexpr (WIN && r == U - 1) store_pw(pw_cur ^ 1);
                         __builtin_amdgcn_sched_barrier(0);
                         wait_lds_and_vmcnt<U == 4 ? CL : 0>();
                         barrier();
@@ -557,7 +563,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
                         if constexpr (t == 3 && k == 0) {
 #pragma unroll
                             for (int jj = 0; jj < TN; jj++) read_c(cbuf((r + 1) % U), jj);
-                            param_words(pring[PW ? 0 : (r + 1) % U], (r + 1) % U, r + 1 < U ? pw_cur : pw_cur ^ 1, sw, bw);
+                            param_words(pring[WIN ? 0 : (r + 1) % U], (r + 1) % U, r + 1 < U ? pw_cur : pw_cur ^ 1, sw, bw);
                         }
                         if constexpr (k < TM) aop[(t + 1) & 1][k] = read_a(abuf(t < 3 ? r & 1 : (r + 1) & 1), (t + 1) & 3, k);
                         // (the last k-step's dequantization waits for the codes just read)
@@ -572,7 +578,7 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
                         }
                         if constexpr (t == 3) {
                             if constexpr (k == 0) {
-                                if constexpr (!PW) load_p(pring[r], i + U);
+                                if constexpr (!WIN) load_p(pring[r], i + U);
                                 else if constexpr (r == 0) load_pw(i0 / U + 1);
                                 __builtin_amdgcn_sched_barrier(0);
                             }
@@ -651,8 +657,8 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     }
 }
 
-// Scale, activation and group-size dispatch of one tile shape.  Group size 16
-// and MXFP4 have no parameter windows, group size 32 always has them.
+// Scale, activation, group-size and parameter-load (pw) dispatch of one tile
+// shape; MXFP4 reads its scales a byte at a time.
 template <int TM, int TN>
 static bool qmm_run_tile(int bits, int gs, int scale_dtype, int x_dtype, bool pw, const QmmArgs& a, int workgroups,
                          hipStream_t st) {
@@ -661,8 +667,10 @@ static bool qmm_run_tile(int bits, int gs, int scale_dtype, int x_dtype, bool pw
         constexpr int B = decltype(bc)::value;
         typedef decltype(stt) ST;
         typedef decltype(xt) XT;
-        if (gs == 16) qmm_mfma_kernel<B, 16, ST, false, XT, TM, TN><<<grid, block, 0, st>>>(a);
-        else if (gs == 32) qmm_mfma_kernel<B, 32, ST, true, XT, TM, TN><<<grid, block, 0, st>>>(a);
+        if (gs == 16 && pw) qmm_mfma_kernel<B, 16, ST, true, XT, TM, TN><<<grid, block, 0, st>>>(a);
+        else if (gs == 16) qmm_mfma_kernel<B, 16, ST, false, XT, TM, TN><<<grid, block, 0, st>>>(a);
+        else if (gs == 32 && pw) qmm_mfma_kernel<B, 32, ST, true, XT, TM, TN><<<grid, block, 0, st>>>(a);
+        else if (gs == 32) qmm_mfma_kernel<B, 32, ST, false, XT, TM, TN><<<grid, block, 0, st>>>(a);
         else if (gs == 64 && pw) qmm_mfma_kernel<B, 64, ST, true, XT, TM, TN><<<grid, block, 0, st>>>(a);
         else if (gs == 64) qmm_mfma_kernel<B, 64, ST, false, XT, TM, TN><<<grid, block, 0, st>>>(a);
         else if (gs == 128 && pw) qmm_mfma_kernel<B, 128, ST, true, XT, TM, TN><<<grid, block, 0, st>>>(a);

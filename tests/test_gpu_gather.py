@@ -17,7 +17,8 @@ import torch
 
 from eredu_amd import EreduError, gather_qmm, gather_qmm_with_mode
 from oracle import oracle as orc
-from tests.fixtures import dev_bf16, dev_param, dev_words, host_f32, synthetic_linear, synthetic_x
+from tests.fixtures import (dev_bf16, dev_param, dev_words, device_random_linear, host_f32, synthetic_linear,
+                            synthetic_x)
 
 pytestmark = pytest.mark.gpu
 
@@ -329,3 +330,28 @@ def test_index_forms_agree_with_the_flat_int32_call(cuda, form):
         other = gather_qmm(xd, *args, None, rhs)
     assert tuple(other.shape) == (R, 1, N)
     assert torch.equal(flat, other)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [16, 32, 64, 128])
+def test_grouped_parameters_at_two_byte_addresses(cuda, gs, bits):
+    """Sorted routes with the bank's scales and biases at element 1 of a larger
+    buffer: bit-equal to the aligned bank (32 and 200 rows per expert: both
+    tiles)."""
+    E, N, K = 4, 256, 1152 if gs < 128 else 1280
+    w, s, b = device_random_linear(E * N, K, gs, bits, seed=gs + bits)
+    w, s, b = (t.view(E, N, -1) for t in (w, s, b))
+
+    def odd(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].view(t.shape)
+
+    g = torch.Generator(device="cuda").manual_seed(gs)
+    for rows in (32, 200):
+        print(f"[case] gather at 2 bytes gs={gs} bits={bits} rows={rows}", flush=True)
+        x = torch.randn((E * rows, 1, K), device="cuda", generator=g).to(torch.bfloat16)
+        ids = torch.arange(E, dtype=torch.int32, device="cuda").repeat_interleave(rows)
+        how = dict(transpose=True, group_size=gs, bits=bits, sorted_indices=True)
+        assert odd(s).data_ptr() % 4 == 2
+        assert torch.equal(gather_qmm(x, w, odd(s), odd(b), None, ids, **how), gather_qmm(x, w, s, b, None, ids, **how))

@@ -14,8 +14,8 @@ import torch
 from eredu_amd import (EreduError, QuantizedLinear, dequantize_with_mode, quantized_matmul, quantized_matmul_batched,
                        quantized_matmul_with_mode)
 from oracle import oracle as orc
-from tests.fixtures import (dev_bf16, dev_param, dev_words, host_bits16, host_f32, synthetic_linear,
-                            synthetic_x)
+from tests.fixtures import (dev_bf16, dev_param, dev_words, device_random_linear, host_bits16, host_f32,
+                            synthetic_linear, synthetic_x)
 
 pytestmark = pytest.mark.gpu
 
@@ -166,6 +166,31 @@ def test_qmm_steps_and_windows(cuda, bits, gs, K, M, N):
 @pytest.mark.parametrize("M,N,K", [(33, 256, 4096), (97, 512, 8320)])
 def test_qmm_split_k_groups(cuda, bits, gs, M, N, K):
     run_bounded(M, N, K, gs, bits, seed=M + gs + bits)
+
+
+def at_odd_element(t):
+    """t's values at a 2-byte aligned address: element 1 of a larger buffer."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.reshape(-1)
+    view = flat[1:].view(t.shape)
+    assert view.is_contiguous() and view.data_ptr() % 4 == 2
+    return view
+
+
+# Scales and biases at 2-byte addresses (views into one parameter buffer): read
+# two bytes at a time, same values, same sums.  64 x 128 tiles with K split and
+# tails, 96 x 128, 128 x 128 and 128 x 256 tiles.
+@pytest.mark.parametrize("bits", [4, 8, 6])
+@pytest.mark.parametrize("gs", [16, 32, 64, 128])
+@pytest.mark.parametrize("M,N,K", [(33, 384, 1152), (77, 14336, 512), (130, 256, 256), (600, 3968, 1024)])
+def test_qmm_parameters_at_two_byte_addresses(cuda, M, N, K, gs, bits):
+    print(f"[case] M={M} N={N} K={K} gs={gs} bits={bits}", flush=True)
+    w, s, b = device_random_linear(N, K, gs, bits, seed=M + gs + bits)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    y = quantized_matmul(x, w, s, b, True, gs, bits)
+    for sv, bv in ((at_odd_element(s), at_odd_element(b)), (s, at_odd_element(b)), (at_odd_element(s), b)):
+        assert torch.equal(quantized_matmul(x, w, sv, bv, True, gs, bits), y)
 
 
 @pytest.mark.parametrize("xdt", [orc.F32, orc.F16])
