@@ -228,8 +228,9 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const __amdgpu_buffer_rsrc_t xr = raw_rsrc(xp, uint32_t(x_rows) * uint32_t(K) * 2u);
     const uint32_t row_bytes = uint32_t(K) * BITS / 8u;  // (the launcher keeps N * row_bytes below 2^31)
     const __amdgpu_buffer_rsrc_t wr = raw_rsrc(wp, uint32_t(N) * row_bytes);
-    const __amdgpu_buffer_rsrc_t sr = raw_rsrc(sp, uint32_t(N) * uint32_t(G) * PB);
-    const __amdgpu_buffer_rsrc_t br = raw_rsrc(bp ? bp : sp, bp ? uint32_t(N) * uint32_t(G) * PB : 0u);
+    const uint32_t p_bytes = uint32_t(N) * uint32_t(G) * PB;
+    const __amdgpu_buffer_rsrc_t sr = raw_rsrc(sp, p_bytes);
+    const __amdgpu_buffer_rsrc_t br = raw_rsrc(bp ? bp : sp, bp ? p_bytes : 0u);
     // Parameter windows in LDS: [buffer][scale, bias][word][column]; a word is
     // two consecutive groups (the first in the low half).
     constexpr int PWW = !WIN ? 1 : GS == 32 ? 2 * U : GS == 64 ? U : U / 2;  // words per column and window
@@ -316,8 +317,14 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     struct PSlot {
         uint32_t s[TN][NPL], b[TN][NPL];
     };
+    // Past the last step the buffers are empty, so that nothing is fetched: a
+    // parameter load touches a cache line per row, and in a split of 4 steps the
+    // 4 requested ahead would double them (group 16, 1024 x 4096, 4-bit, 8
+    // splits: M = 64 13.6 us with those, 13.0 without).
     auto load_p = [&](PSlot& S, int i) __attribute__((always_inline)) {
         const uint32_t kp = __builtin_amdgcn_readfirstlane(uint32_t(chunk_k0(i) / GS) * PB);
+        const __amdgpu_buffer_rsrc_t sr = raw_rsrc(sp, i < steps ? p_bytes : 0u);
+        const __amdgpu_buffer_rsrc_t br = raw_rsrc(bp ? bp : sp, bp && i < steps ? p_bytes : 0u);
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             if constexpr (MX) {

@@ -10,7 +10,7 @@ namespace eq {
 // below group size 64) and, with a split of K, splits that start at an even
 // group.  A view at an odd element of a larger buffer is only 2-byte aligned;
 // such a call reads its parameters two bytes at a time instead (4-bit group 32,
-// 14336 x 4096: M = 512 86 us against 67 with windows, M = 64 30 against 23).
+// 14336 x 4096: M = 512 80 us against 67 with windows, M = 64 28 against 23).
 inline bool qmm_param_words(int gs, int K, int cps, const void* s, const void* b) {
     if ((reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(b)) % 4 != 0) return false;  // (no biases: null)
     return gs == 16 || gs == 32 || (gs == 64 && (K / 64) % 2 == 0 && cps % 2 == 0) ||
