@@ -4,7 +4,6 @@
 #include <mutex>
 
 #include "qmm_kernel.hpp"
-#include "qmm_plan.hpp"
 
 namespace eq {
 
@@ -46,87 +45,6 @@ static int qmm_cu_count() {
     return v;
 }
 
-// Tile shape and split of K of one launch.  Up to 128 rows: one of the narrow
-// tiles, by qmm_plan_few_rows.  Above: 128 x 256 tiles when there are at least
-// 3/4 as many as CUs, or when K split to fill the CUs still leaves each split
-// 32 chunks or more; otherwise 64 x 128 tiles (four times as many, each
-// dequantized code used by 64 rows instead of 128) when the large tiles would
-// split K 8 ways or more, or at group sizes with parameter windows (whose
-// dequantization is the cheapest per code), unless the 128 x 128 tiles below
-// take the call.  K is split so that the grid fills the CUs without exceeding
-// them (a second round would double the time), at least 8 chunks per split (4
-// per K-group).  Measured with weights rotated from HBM, 4-bit: M = 512, 4096 x
-// 4096, the large tiles' 4 splits against the 128 x 128 tiles' two: group 32
-// 43.5 -> 32.0 us, group 128 40.0 -> 29.0; at group 16 (the 2/3/5/6-bit
-// re-packed codes included) the small tiles' per-code work made them 2-8 %
-// slower there.  M = 96, 4096 x 4096, group 32, 64 x 128 tiles and 4 splits
-// against 96 x 128 and 8: 15.4 against 19.7 us; M = 77, 14336 x 4096, 96 x 128
-// against 128 x 128 tiles, both split twice: 24.8 against 26.2.
-struct QmmPlan {
-    int tm, tn;  // 32-row and 128-column blocks of a tile
-    int mtiles, ntiles, splits;
-};
-static int qmm_splits(int tiles, int slots, int nchunks) {
-    int s = slots / (tiles > 0 ? tiles : 1);
-    s = s > nchunks / 8 ? nchunks / 8 : s;
-    return s < 1 ? 1 : s;
-}
-// The cheapest plan of at most 128 rows, in microseconds: a workgroup walks
-// its steps of two chunks in `step` each (64, 96 and 128 rows measured at
-// 0.70, 0.87 and 1.0 us, whether or not a second workgroup shares the CU)
-// after 5 us of launch, first loads and reduction; partials are written and
-// read back at 4 MB/us, and their reduction is a launch of 2.5 us.  Where the
-// 64 x 128 tiles cover more than half the CUs and K is short, K is split only if
-// the pieces stay at 24 chunks, fill 3/4 of the CUs and write partials of at
-// most twice the weight bytes: such calls otherwise need no workspace, and may
-// be captured without an eager call before.
-static QmmPlan qmm_plan_few_rows(int M, int N, int cu, int nchunks, bool may_split) {
-    QmmPlan best{};
-    double least = 0;
-    const bool short_k = qmm_splits((M + 63) / 64 * ((N + 127) / 128), cu, nchunks) == 1 &&
-                         nchunks / qmm_splits((N + 255) / 256, cu, nchunks) < 32;
-    const double step[3] = {0.70, 0.87, 1.0};
-    for (int tm = 2; tm <= 4; tm++) {
-        const int mt = (M + 32 * tm - 1) / (32 * tm), nt = (N + 127) / 128;
-        const int most = may_split ? qmm_splits(mt * nt, cu, nchunks) : 1;
-        for (int s = 1; s <= most; s++) {
-            if (s > 1 && short_k &&
-                (nchunks / s < 24 || 4 * mt * nt * s < 3 * cu || int64_t(s) * M * 4 > int64_t(nchunks) * kBK))
-                continue;
-            const int rounds = (mt * nt * s + cu - 1) / cu, steps = (nchunks + 2 * s - 1) / (2 * s);
-            const double us = rounds * (5.0 + steps * step[tm - 2]) + (s > 1 ? 2.5 + 8.0 * s * M * N / 4e6 : 0.0);
-            if (!best.tm || us < least) least = us, best = QmmPlan{tm, 1, mt, nt, s};
-        }
-    }
-    return best;
-}
-static QmmPlan qmm_plan(int M, int N, int K, int gs, int bits, bool may_split) {
-    const int cu = qmm_cu_count(), nchunks = K / kBK;
-    if (M <= 128) return qmm_plan_few_rows(M, N, cu, nchunks, may_split);
-    QmmPlan p{4, 2, 0, 0, 1};
-    const int big = ((M + 127) / 128) * ((N + 255) / 256);
-    const int big_splits = may_split ? qmm_splits(big, cu, nchunks) : 1;
-    const bool big_ok = 4 * big >= 3 * cu || nchunks / big_splits >= 32;
-    const bool small_ok = big_splits >= 8 || gs >= 32;
-    if (!big_ok && small_ok) p.tm = 2, p.tn = 1;
-    // 128 x 128 tiles (group sizes with parameter windows) in place of the
-    // small tiles, or of large tiles that split K, when their own split leaves
-    // each piece at least 24 chunks, fills 3/4 of the CUs and writes f32
-    // partials of at most twice the weight bytes: every code then feeds 128
-    // rows, as in the large tile, with twice the large tile's workgroups.
-    if (may_split && gs >= 32 && (p.tm == 2 || big_splits > 1)) {
-        const int mid = ((M + 127) / 128) * ((N + 127) / 128);
-        const int ms = qmm_splits(mid, cu, nchunks);
-        const bool fills = 4 * mid * ms >= 3 * cu;
-        const bool long_k = nchunks / ms >= 24;
-        const bool partials_ok = ms == 1 || double(ms) * M * N * 4.0 <= 2.0 * double(N) * double(K) * bits / 8.0;
-        if (fills && long_k && partials_ok && (p.tm == 2 || ms < big_splits)) p.tm = 4, p.tn = 1;
-    }
-    p.mtiles = (M + 32 * p.tm - 1) / (32 * p.tm), p.ntiles = (N + 128 * p.tn - 1) / (128 * p.tn);
-    p.splits = may_split ? qmm_splits(p.mtiles * p.ntiles, cu, nchunks) : 1;
-    return p;
-}
-
 // The types of a launch: code bits, group size, scale (EQ_DTYPE_U8: MXFP4) and activation types.
 struct QmmTypes {
     int bits, gs, scale_dtype, x_dtype;
@@ -147,7 +65,7 @@ static bool launch_qmm_piece(const QmmTypes& t, uint16_t* y, int ldy, const uint
     QmmArgs a{};
     a.y = y, a.x = x, a.w = w, a.s = static_cast<const uint16_t*>(s), a.b = static_cast<const uint16_t*>(b);
     a.M = M, a.N = N, a.K = K, a.ldy = ldy;
-    const QmmPlan plan = qmm_plan(M, N, K, t.gs, t.bits, may_split);
+    const QmmPlan plan = qmm_plan(M, N, K, t.gs, t.bits, may_split, qmm_cu_count());
     a.mtiles = plan.mtiles, a.ntiles = plan.ntiles;
     const int tiles = a.mtiles * a.ntiles, nchunks = K / kBK;
     int splits = plan.splits;
@@ -413,7 +331,7 @@ static bool launch_qmm_odd_t(const QmmTypes& t, uint16_t* y, const uint16_t* x, 
     nc = nc > N ? N : nc;
     const size_t code_bytes = (size_t(nc) * size_t(K) + 255) & ~size_t(255);
     // room after the codes for the split-K partials of a slice the planner would split
-    const int splits = qmm_plan(M, int(nc), K, gs, 8, true).splits;
+    const int splits = qmm_plan(M, int(nc), K, gs, 8, true, qmm_cu_count()).splits;
     const size_t part_bytes = splits > 1 ? size_t(splits) * size_t(M) * size_t(nc) * 4u : 0;
     size_t want = code_bytes + part_bytes;
     char* base = static_cast<char*>(ws_acquire(src, want, st));

@@ -61,12 +61,12 @@
 #include <utility>
 
 #include "eq_common.hpp"
+#include "qmm_plan.hpp"
 
 namespace eq {
 
 typedef uint32_t q_u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 128, kBN = 256, kBK = 64;  // the default tile (rows, columns) and the K chunk
 constexpr int kQmmThreads = 512;               // two K-groups of 4 waves
 
 // Steps of codes a kernel variant holds in LDS ahead of their use, which is
