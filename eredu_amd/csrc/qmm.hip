@@ -164,8 +164,8 @@ __device__ __forceinline__ int lower_bound_i32(const int32_t* __restrict__ a, in
 // Prepares a grouped launch.  Workgroup 0: sorted expert indices -> the tile
 // list; expert e owns rows [lower_bound(e), lower_bound(e + 1)) and takes
 // ceil(rows / bm) entries {e, first, rows, bm t}, experts in passes of 1024
-// with a block scan of the entry counts; entries at or past `cap` are dropped
-// and the list's remaining entries are marked unused.  The indices are searched
+// with a block scan of the entry counts; entries at or past `cap` are dropped,
+// and out[cap] receives how many there are.  The indices are searched
 // in LDS where they fit (from memory a search is a chain of a dozen trips).
 // The other workgroups meanwhile clear y (rows of no expert stay zero), n bf16
 // values, n a multiple of 4, y 8-byte aligned.
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(1024) void qmm_group_prepare(int4* __restrict__ out
         if (tid == last) carry += scan[last];
         __syncthreads();
     }
-    for (int i = carry + tid; i < cap; i += 1024) out[i] = make_int4(-1, 0, 0, 0);
+    if (tid == 0) out[cap] = make_int4(carry < cap ? carry : cap, 0, 0, 0);
 }
 
 // xg[b] = x[lhs[b]] (K bf16 per row, 16-byte copies); an out-of-range index
@@ -232,22 +232,25 @@ __global__ __launch_bounds__(256) void qmm_gather_rows(uint16_t* __restrict__ xg
 static bool launch_qmm_grouped_t(const QmmTypes& t, uint16_t* y, const uint16_t* x, const uint32_t* w, const void* s, const void* b,
                                  const int32_t* lhs, const int32_t* rhs, int batch, int64_t x_batches, int experts,
                                  int N, int K, hipStream_t st, const WsSource* src = nullptr) {
-    // Tiles by the mean number of rows per expert: 64 x 128 up to 96 (two such
-    // workgroups share a CU), 128 x 256 above.  Measured, the SwiGLU of a prompt's
-    // sorted routes, 64 x 128 against 128 x 256 tiles: 128 experts of 768 x 2048 at
-    // 4 rows each 148 / 197 us, at 32 rows 218 / 236, 64 experts of 1024 x 2048 at
-    // 64 rows 178 / 209, at 128 rows 273 / 271; 8 experts of 7168 x 4096 at 128 rows
-    // 408 / 372.  (With 128 x 256 tiles, y cleared and the rows gathered by launches
-    // of their own and the indices searched in memory, before: 276 us at 32 rows.)
+    // Tiles by the mean number of rows per expert: 64 x 128 up to 64 rows (two such
+    // workgroups of 4-bit codes share a CU), 128 x 256 above; with 8-bit codes (one
+    // to a CU) and at group size 16 (more work per code) up to 40.  Time of the 64
+    // x 128 tiles over that of the 128 x 256 ones, geometric mean of six banks of 8 to
+    // 128 experts: 4-bit group 64 at 40 / 56 / 64 / 80 rows 0.75 / 0.90 / 0.98 /
+    // 1.07, group 32 0.78 / 0.94 / 1.02 at 64, group 16 0.78 / 1.01 / 1.11; 8-bit
+    // group 64 at 40 / 48 / 64 rows 0.87 / 1.09 / 1.19.  Routes on few of the experts
+    // fill the tiles they take, at these means and above (128 experts of 768 x 2048,
+    // 16 rows in the mean, all on two: 20 / 33 us; 64 rows: 47 / 42).
     const int mean = batch / (experts > 0 ? experts : 1);
-    const int tm = mean <= 96 ? 2 : 4, tn = mean <= 96 ? 1 : 2, bm = 32 * tm;
+    const bool small = mean <= (t.bits == 4 && t.gs >= 32 ? 64 : 40);
+    const int tm = small ? 2 : 4, tn = small ? 1 : 2, bm = 32 * tm;
     const int cap = experts + (batch + bm - 1) / bm;  // sum over experts of ceil(rows / bm)
     // one launch with 32-bit offsets: each expert's codes below 2^31 bytes, and
     // the rows of x, which are otherwise gathered first
     if (int64_t(N) * K * t.bits / 8 >= (int64_t(1) << 31) || int64_t(batch) * K * 2 >= (int64_t(1) << 31)) return false;
     const bool direct = x_batches * int64_t(K) * 2 < (int64_t(1) << 31);
     const size_t xg_bytes = direct ? 0 : (size_t(batch) * size_t(K) * 2u + 255u) & ~size_t(255);
-    void* ws = ws_acquire(src, xg_bytes + size_t(cap) * sizeof(int4), st);
+    void* ws = ws_acquire(src, xg_bytes + size_t(cap + 1) * sizeof(int4), st);
     if (!ws) return false;
     uint16_t* xg = reinterpret_cast<uint16_t*>(ws);
     int4* list = reinterpret_cast<int4*>(reinterpret_cast<char*>(ws) + xg_bytes);
@@ -261,7 +264,7 @@ static bool launch_qmm_grouped_t(const QmmTypes& t, uint16_t* y, const uint16_t*
     a.mtiles = cap, a.ntiles = (N + 128 * tn - 1) / (128 * tn), a.splits = 1, a.cps = K / kBK;
     a.groups = list;
     a.lhs = direct ? lhs : nullptr, a.x_rows = direct ? int(x_batches) : batch;
-    return qmm_run(tm, tn, t, a, a.mtiles * a.ntiles, st);
+    return qmm_run(tm, tn, t, a, (a.mtiles * a.ntiles + 7) / 8 * 8, st);  // (an eighth for each XCD, rounded up)
 }
 
 bool launch_qmm_grouped(int bits, int gs, int scale_dtype, uint16_t* y, const uint16_t* x, const uint32_t* w,

@@ -135,11 +135,11 @@ struct QmmArgs {
     const uint16_t* s;
     const uint16_t* b;  // may be null
     int M, N, K, ldy, mtiles, ntiles, splits, cps;  // cps: chunks per split; ldy: y row stride
-    // Grouped (routed experts, no split K): row tile tm of the grid is entry
-    // groups[tm] = {expert, first row, rows, row offset} of a device-built
-    // list; x and y rows [first, first + rows) belong to the expert, whose
-    // weights, scales and biases follow the previous expert's.  An expert
-    // below zero marks an unused entry.  Null: one plain problem.
+    // Grouped (routed experts, no split K): row tile tm is entry groups[tm] =
+    // {expert, first row, rows, row offset} of a device-built list; x and y rows
+    // [first, first + rows) belong to the expert, whose weights, scales and biases
+    // follow the previous expert's.  Entry groups[mtiles] holds how many of the
+    // mtiles are in use.  Null: one plain problem.
     const int4* groups;
     // Grouped: y row r multiplies x row lhs[r] (null: row r, or row 0 of a
     // single one) of x_rows; an index outside them reads zeros.
@@ -160,8 +160,9 @@ struct QmmArgs {
 // the workgroup's tile is 32 TM rows x 128 TN columns (4 x 2: 128 x 256, the
 // default; 4 x 1 and 2 x 1: 128 x 128 and 64 x 128, for outputs with too few
 // large tiles to fill the GPU, which then need no split of K or fewer splits;
-// 3 x 1: 96 x 128).  A 2 x 1 workgroup leaves room for a second one on its CU
-// (72 KiB of LDS, 80 registers): routed experts of 32 rows 252 -> 218 us.
+// 3 x 1: 96 x 128).  A 2 x 1 workgroup of 4-bit codes leaves room for a second
+// one on its CU (64-80 KiB of LDS, 80 registers; with 8-bit codes 96-112 KiB):
+// routed experts of 32 rows 252 -> 218 us.
 template <int BITS, int GS, typename ST, bool PW, typename XT, int TM, int TN>
 __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, TM == 2 ? 4 : 2))) void qmm_mfma_kernel(
     const QmmArgs args) {
@@ -187,10 +188,20 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     int M = args.M;
 
     // Tile and split of this workgroup: the workgroups of one XCD (id % 8)
-    // take a contiguous run of row-major tiles, i.e. few row blocks of x.
+    // take a contiguous run of row-major tiles, i.e. few row blocks of x.  Grouped:
+    // an eighth of the tiles in use; with runs over the whole list, which must
+    // have room for a part tile per expert, the last XCDs got none (8 experts of
+    // 7168 x 4096, 8-bit, 128 routes to two of them 77 -> 29 us, to all 100 -> 75;
+    // 128 experts of 768 x 2048, 4-bit, 4096 routes 60 -> 45).
     const int T = args.mtiles * args.ntiles * args.splits;
     int bid = blockIdx.x;
-    if ((T & 7) == 0) bid = (bid & 7) * (T >> 3) + (bid >> 3);
+    if (args.groups) {
+        const int used = args.groups[args.mtiles].x * args.ntiles, run = (used + 7) >> 3, at = bid >> 3;
+        bid = (bid & 7) * run + at;
+        if (at >= run || bid >= used) return;  // (the whole workgroup, before any barrier)
+    } else if ((T & 7) == 0) {
+        bid = (bid & 7) * (T >> 3) + (bid >> 3);
+    }
     const int split = bid % args.splits, tile = bid / args.splits;
     const int tm = tile / args.ntiles, tn = tile % args.ntiles;
     int m0 = tm * BM;
@@ -203,7 +214,6 @@ __global__ __launch_bounds__(kQmmThreads) __attribute__((amdgpu_waves_per_eu(2, 
     int first = 0, x_rows = M;
     if (args.groups) {
         const int4 gd = args.groups[tm];
-        if (gd.x < 0) return;  // unused entry: the whole workgroup leaves before any barrier
         first = gd.y, x_rows = args.x_rows;
         yp += int64_t(gd.y) * args.ldy;
         M = gd.z;

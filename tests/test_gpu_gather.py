@@ -286,13 +286,15 @@ def test_grouped_and_per_route_paths_on_a_mixtral_like_layout(cuda):
         check(y, y_ref, out_is_bf16=True)
 
 
-@pytest.mark.parametrize("R,E,lhs_kind", [(64, 32, "none"), (768, 8, "picked"), (784, 8, "picked"), (300, 4, "one"),
+@pytest.mark.parametrize("R,E,lhs_kind", [(64, 32, "none"), (512, 8, "picked"), (520, 8, "picked"),
+                                          (768, 8, "picked"), (784, 8, "picked"), (300, 4, "one"),
                                           (8200, 128, "picked")])
 def test_grouped_tile_choice_and_row_sources(cuda, R, E, lhs_kind):
-    """Means of 2, 96 (the last 64-row tiles), 98 and 75 rows per expert, more
-    routes than the prepare kernel holds in LDS; x rows read in place through
-    lhs (out-of-range ones read zeros), row by row, or one row for all; the
-    first and last routes outside the bank (zero rows)."""
+    """Means of 2 and 64 rows per expert (64-row tiles, the last mean that takes
+    them), of 65 to 98 (128-row tiles), more routes than the prepare kernel holds
+    in LDS; x rows read in place through lhs (out-of-range ones read zeros), row
+    by row, or one row for all; the first and last routes outside the bank (zero
+    rows)."""
     from eredu_amd import gather_qmm
 
     N, K, gs, bits = 128, 128, 64, 4
@@ -355,3 +357,14 @@ def test_grouped_parameters_at_two_byte_addresses(cuda, gs, bits):
         how = dict(transpose=True, group_size=gs, bits=bits, sorted_indices=True)
         assert odd(s).data_ptr() % 4 == 2
         assert torch.equal(gather_qmm(x, w, odd(s), odd(b), None, ids, **how), gather_qmm(x, w, s, b, None, ids, **how))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,picks", [(128, [13]), (128, [0, 15]), (384, [3, 4, 9]), (1408, [15])])
+@pytest.mark.parametrize("rows", [48, 700])
+def test_grouped_routes_on_few_experts(cuda, bits, N, picks, rows):
+    """Most of 16 experts without routes: fewer tiles in use than XCDs, counts
+    that eight does not divide, and an unused rest of the list; both tiles."""
+    E, K = 16, 256
+    rhs = np.sort(np.resize(picks, rows)).astype(np.int32)
+    run(E, N, K, 64, bits, None, rhs, Bx=rows, seed=N + rows, sorted_indices=True)
