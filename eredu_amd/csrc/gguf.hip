@@ -395,10 +395,9 @@ __device__ __forceinline__ uint32_t lds_half(const uint8_t* b, int o) {
 // alignment in LDS, where the compiler would merge the reads into wide
 // unaligned ones, which the LDS serves with many stalls (Q6_K linear, 128256 x
 // 4096, M = 1: 62 of 74 M busy LDS cycles were such stalls): there the words
-// around the bytes are read aligned and shifted (that call 161 -> 141 us,
-// 4096 x 14336 23.9 -> 20.9, the Q6_K prefill's re-pack with its product at M =
-// 512, 4096 x 4096, 58.5 -> 50.7 with the product's own change).  The third of
-// them is read only when the bytes reach into it.
+// around the bytes are read aligned and shifted (32768 x 4096 42.8 -> 34.9 us,
+// 4096 x 14336 21.8 -> 19.0).  The third of them is read only when the bytes
+// reach into it.
 template <int T, bool ALIGNED>
 __device__ __forceinline__ void lds_8b(const uint8_t* p, uint32_t& lo, uint32_t& hi) {
     if constexpr (KQuant<T>::bytes % 4 == 0 || !ALIGNED) {
@@ -923,6 +922,28 @@ __global__ __launch_bounds__(256) void q4k_linear(uint16_t* __restrict__ y, cons
 constexpr int kKqStageVec = 8;  // 16-byte pieces per lane of one staged row group
 constexpr int64_t kKqXLds = 40 * 1024;  // LDS per workgroup up to which x is staged as well
 
+// Whether one activation row is staged in LDS beside the weight rows: row groups
+// per workgroup (up to 4) times K must pay for staging it (~0.5 us).  Times with it
+// over times without at 1.1 / 2 / 4 groups per workgroup: Q5_1 K = 1024 1.07 / 1.04
+// / 0.97, 2048 0.99 / 0.96 / 0.88; Q6_K 2048 1.04 / 1.00 / 1.00, 4096 0.99 / 0.95 /
+// 0.95; Q5_K 2048 1.01 / 1.02 / 0.97, 4096 0.99 / 0.96 / 0.93; IQ4_NL 2048 1.05 /
+// 1.03 / 1.00, 4096 1.07 / 1.01 / 0.98, 8192 1.00 / 0.99 / 0.96.
+inline bool kq_stage_x(int ggml_type, int64_t K, int64_t groups, int64_t workgroups) {
+    const int64_t least = ggml_type == EQ_GGML_Q5_1   ? 3400
+                          : ggml_type == EQ_GGML_Q6_K ? 5000
+                          : ggml_type == EQ_GGML_Q5_K ? 6200
+                                                      : 16000;
+    const int64_t capped = groups < 4 * workgroups ? groups : 4 * workgroups;
+    return groups > workgroups && K >= (ggml_type == EQ_GGML_Q5_1 ? 1024 : 2048) && K * capped >= least * workgroups;
+}
+
+// Whether the codes are read from LDS as aligned words (lds_8b).  Q6_K at K >
+// 1024; at shorter rows, which leave lanes idle, the shifts cost more than the
+// stalls (32768 x 512 18.3 against 15.9 us, x 1024 18.5 / 18.0, x 1536 19.1 /
+// 20.9).  IQ4_NL never: its level conversions leave no room for them (32768 x 4096
+// 29.6 against 28.7, 4096 x 14336 15.5 / 15.1).
+inline bool kq_aligned_words(int ggml_type, int64_t K) { return ggml_type == EQ_GGML_Q6_K && K > 1024; }
+
 // Persistent workgroups walk row groups grp, grp + gridDim.x, ...; a full
 // group on a 16-byte-aligned payload is fetched into registers one group
 // ahead (its loads in flight while the current group is multiplied), a
@@ -933,9 +954,9 @@ constexpr int64_t kKqXLds = 40 * 1024;  // LDS per workgroup up to which x is st
 // 64 lanes of a unit step read consecutive pieces.  From memory the same reads
 // are 64 bytes apart, a cache line per two lanes, and every weight row costs
 // 256 cycles of the texture unit per 64 units: with the codes read aligned
-// that unit was busy for 93 % of the launch.  M = 1 at K = 4096: Q6_K 14336 rows
-// 19.9 -> 18.8 us, 128256 rows 141 -> 136, Q5_K 32768 rows 34.7 -> 32.0.
-template <int T, bool BIG, bool MANY, int W, bool XL>
+// that unit was busy for 93 % of the launch (kq_stage_x: where it pays).
+// WORDS: lds_8b's aligned words (kq_aligned_words).
+template <int T, bool BIG, bool MANY, int W, bool XL, bool WORDS>
 __global__ __launch_bounds__(64 * W) void kq_linear(uint16_t* __restrict__ y, const uint16_t* __restrict__ x,
                                                     const uint8_t* __restrict__ raw, int M, int N, int K, int R,
                                                     bool vec_ok, ExpertSel sel) {
@@ -1018,9 +1039,7 @@ __global__ __launch_bounds__(64 * W) void kq_linear(uint16_t* __restrict__ y, co
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     uint32_t c0, c1;
-                    // (with several activation rows the x reads set the time, and the
-                    // shifts only add to it: 4096 x 14336, M = 8, 79.0 against 81.9 us)
-                    kq_codes8<T, BIG, !MANY>(b, uu, 8 * q, c0, c1);
+                    kq_codes8<T, BIG, WORDS>(b, uu, 8 * q, c0, c1);
                     if constexpr (P::levels) {
                         // level + 128 (up to 241: exact in bf16, past the 0x43 trick's
                         // range) converted per byte
@@ -1956,10 +1975,9 @@ int native_linear_run(void* y, const void* x, const uint8_t* raw, int ggml_type,
                     for (int64_t m0 = 0; m0 < M; m0 += mcap) {
                         const int mc = int(M - m0 < mcap ? M - m0 : mcap);
                         // x in LDS for one activation row, while the four workgroups of a CU
-                        // still fit (K = 14336: 20.9 -> 26.6 us with fewer) and walk more than
-                        // one group each (1024 x 4096: 6.2 -> 6.4)
+                        // still fit (K = 14336: 20.9 -> 26.6 us with fewer)
                         const int64_t with_x = rows_lds + (mc * sx_row + 15) / 16 * 16 + int64_t(mc) * K * 2;
-                        const bool xl = mc == 1 && with_x <= kKqXLds && groups > cap;
+                        const bool xl = mc == 1 && with_x <= kKqXLds && kq_stage_x(T, K, groups, cap);
                         const int lds = int(xl ? with_x : rows_lds + mc * sx_row);
                         auto go = [&](auto kernel) {
                             if (lds > 65536)
@@ -1970,9 +1988,14 @@ int native_linear_run(void* y, const void* x, const uint8_t* raw, int ggml_type,
                                                                   static_cast<const uint16_t*>(x) + m0 * K, raw, mc,
                                                                   int(N), int(K), R, vec_ok, sel);
                         };
-                        if (xl) go(kq_linear<T, B, false, W, true>);
-                        else if (mc == 1) go(kq_linear<T, B, false, W, false>);
-                        else go(kq_linear<T, B, true, W, false>);
+                        // aligned words for one activation row (with several the x reads set the
+                        // time, and the shifts only add to it: Q6_K 4096 x 14336, M = 8, 79.0
+                        // against 81.9 us); rows long enough for x in LDS are for them too
+                        constexpr bool Q6 = T == EQ_GGML_Q6_K;
+                        if (xl) go(kq_linear<T, B, false, W, true, Q6>);
+                        else if (mc == 1 && Q6 && kq_aligned_words(T, K)) go(kq_linear<T, B, false, W, false, Q6>);
+                        else if (mc == 1) go(kq_linear<T, B, false, W, false, false>);
+                        else go(kq_linear<T, B, true, W, false, false>);
                     }
                 }
             }))

@@ -79,14 +79,35 @@ def test_native_linear_big_endian_and_unaligned_payload(cuda, ty):
     run_case(ty, 200, 2048, 1, seed=8, offset=2)
 
 
-# One activation row staged in LDS beside the rows: more than four row groups
-# per CU (8 rows each), the last one partial; odd and even superblock counts
-# (Q6_K rows then start at 2-byte and 4-byte offsets); both byte orders.
+# More than four row groups per CU (8 rows each), the last one partial; odd and
+# even superblock counts (Q6_K rows then start at 2-byte and 4-byte offsets; codes
+# read as they lie at K = 256, as aligned words above 1024); both byte orders.
 @pytest.mark.parametrize("ty", [T.Q5_1, T.Q5K, T.Q6K])
 @pytest.mark.parametrize("K,endian", [(256, G.Endian.Little), (1280, G.Endian.Big), (2048, G.Endian.Little)])
 def test_native_linear_staged_row(cuda, ty, K, endian):
     print(f"[case] native {ty.name} N=8205 K={K} M=1 {endian!r}", flush=True)
     run_case(ty, 8205, K, 1, seed=K + int(ty), endian=endian)
+
+
+# One activation row staged in LDS beside the rows (at least 4 row groups per
+# workgroup and the shortest such K of each type; Q6_K also at an odd superblock
+# count), the last group partial: bit-equal to slices of 4096 rows, one group per
+# workgroup, which read x from memory.
+@pytest.mark.parametrize("ty,K,endian", [(T.Q5_1, 1024, G.Endian.Little), (T.Q5K, 2048, G.Endian.Little),
+                                         (T.Q6K, 2048, G.Endian.Little), (T.Q6K, 2304, G.Endian.Big),
+                                         (T.IQ4NL, 4096, G.Endian.Little), (T.IQ4XS, 4096, G.Endian.Little)])
+def test_native_linear_row_in_lds_equals_slices(cuda, ty, K, endian):
+    print(f"[case] native {ty.name} N=32781 K={K} M=1 {endian!r}", flush=True)
+    N, (vals, nbytes) = 32781, ty.block_and_bytes()
+    raw = synthetic_blocks(int(ty), N * K // vals, seed=K)
+    raw = dev_u8(_to_big_endian(int(ty), raw) if endian == G.Endian.Big else raw)
+    row = K // vals * nbytes
+    x = dev_bf16(synthetic_x(1, K, 3))
+    y = G.linear(x, G.TensorDescriptor("w", [K, N], ty, raw.numel()), raw, endian)
+    for n0 in range(0, N, 4096):
+        n = min(4096, N - n0)
+        part = raw[n0 * row:(n0 + n) * row]
+        assert torch.equal(y[:, n0:n0 + n], G.linear(x, G.TensorDescriptor("w", [K, n], ty, part.numel()), part, endian))
 
 
 def test_native_q6k_row_longer_than_64k(cuda):
