@@ -215,7 +215,7 @@ def native_closed_form(ty, raw, N, K):
 
 # Prefill (M > 8): the slice's blocks converted to the affine triple in the
 # workspace and multiplied on the matrix cores (4/8-bit directly, 5/6-bit
-# through the byte re-pack); M = 12, 17 and 130 leave partial 128-row tiles.
+# through the byte re-pack); M = 12, 17 and 130 leave partial tiles of rows.
 @pytest.mark.parametrize("ty,K", [(T.Q4K, 2048), (T.Q5K, 1024), (T.Q6K, 2048), (T.Q5_1, 1024), (T.Q8_0, 2048)])
 @pytest.mark.parametrize("M", [12, 17, 64, 130])
 def test_native_linear_prefill(cuda, ty, K, M):

@@ -100,17 +100,16 @@ def test_qmm_f16_scales(cuda):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 448])
 def test_qmm_pipeline_depths(cuda, bits, K):
-    # 1..7 chunks of 64 in one workgroup (too few to split K): every position
-    # of the three-slot load ring, including the wrap-around
+    # 1..7 chunks of 64 in one workgroup (too few to split K): 1 to 4 steps of
+    # two chunks, the last with one where the count is odd
     run_case(40, 256, K, 64, bits, seed=K + bits)
 
 
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("M,gs", [(65, 64), (100, 64), (100, 32)])
 def test_qmm_tiles_ragged(cuda, bits, M, gs):
-    # N = 384: three 64 x 128 tiles (group 64) or two 128 x 256 tiles, the
-    # second half past N (group 32, which keeps the large tile); M not a
-    # multiple of either tile height; K split 4 ways in both plans
+    # two rows of three 64 x 128 tiles, M not a multiple of the tile's height;
+    # K split 4 ways
     run_case(M, 384, 2048, gs, bits, seed=M + gs + bits)
 
 
@@ -128,23 +127,33 @@ def test_qmm_mid_tiles_ragged(cuda, bits, M, N, K):
 
 @pytest.mark.parametrize("bits", [4, 8])
 def test_qmm_split_k(cuda, bits):
-    # 6 output tiles, 32 chunks: K split 8 ways, partial tiles summed in order
+    # 20 tiles of 64 x 128, 32 chunks: K split 4 ways, partial tiles summed in order
     run_case(300, 512, 2048, 64, bits, seed=bits + 77)
 
-def run_bounded(M, N, K, gs, bits, seed):
+
+def run_bounded(M, N, K, gs, bits, seed, f16=False):
     """A prefill product against the f64 one, elementwise within what its
-    roundings allow: each weight s*q + b rounds once to bf16 (2^-9 relative)
-    and the products add up in f32 (at most K 2^-24 of their magnitudes, below
-    2^-11 here), so |err| <= (2^-9 + 2^-11) sum |x w| + 1/2 ulp_bf16(y)."""
-    print(f"[case] M={M} N={N} K={K} gs={gs} bits={bits}", flush=True)
+    roundings allow: each weight s*q + b rounds once to the activation type (half an
+    ulp: r = 2^-8 of its magnitude at most with bf16's 8 significant bits, 2^-11
+    with f16's 11, or 2^-25 below f16's normal range) and the products add up in
+    f32 (at most K 2^-24 of their magnitudes); the output rounds once: |err| <= (r +
+    K 2^-24) sum |x w| (+ 2^-25 sum |x|) + r |y| (+ 2^-25)."""
+    print(f"[case] M={M} N={N} K={K} gs={gs} bits={bits} f16={f16}", flush=True)
     w, s, b = synthetic_linear(N, K, gs, bits, seed, scale_dtype=orc.BF16)
     xb = synthetic_x(M, K, seed + 1)
-    y = host_f32(quantized_matmul(dev_bf16(xb), dev_words(w), dev_bf16(s), dev_bf16(b), transpose=True, group_size=gs,
+    x = orc.bf16_bits_to_f32(xb)
+    if f16:
+        x = x.astype(np.float16).astype(np.float32)
+    xd = dev_param(x.astype(np.float16).view(np.uint16), orc.F16) if f16 else dev_bf16(xb)
+    y = host_f32(quantized_matmul(xd, dev_words(w), dev_bf16(s), dev_bf16(b), transpose=True, group_size=gs,
                                   bits=bits)).astype(np.float64)
-    x = orc.bf16_bits_to_f32(xb).astype(np.float64)
+    x = x.astype(np.float64)
     W = orc.affine_dequant_f32(w, s, b, orc.BF16, N, K, gs, bits).reshape(N, K).astype(np.float64)
     ref = x @ W.T
-    bound = (2.0 ** -9 + 2.0 ** -11) * (np.abs(x) @ np.abs(W).T) + 2.0 ** -9 * np.maximum(np.abs(y), np.abs(ref))
+    r = 2.0 ** -11 if f16 else 2.0 ** -8
+    bound = (r + K * 2.0 ** -24) * (np.abs(x) @ np.abs(W).T) + r * np.maximum(np.abs(y), np.abs(ref))
+    if f16:
+        bound += 2.0 ** -25 * np.abs(x).sum(axis=1, keepdims=True) + 2.0 ** -25
     worst = float((np.abs(y - ref) / bound).max())
     assert worst <= 1.0, f"max err / bound = {worst:.3f}"
 
@@ -168,6 +177,26 @@ def test_qmm_split_k_groups(cuda, bits, gs, M, N, K):
     run_bounded(M, N, K, gs, bits, seed=M + gs + bits)
 
 
+# 96 x 128 tiles (65 to 96 rows of 4224 and more columns): split 4 and 3 ways and,
+# with more than half as many tiles as CUs, not at all; whole tiles of rows and
+# part ones, an odd chunk count, rows of an odd number of groups.
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs,f16", [(16, False), (32, False), (64, False), (128, False), (64, True)])
+@pytest.mark.parametrize("M,N,K", [(66, 4224, 2048), (96, 5504, 2112), (77, 16512, 192)])
+def test_qmm_96_row_tiles(cuda, M, N, K, gs, f16, bits):
+    run_bounded(M, N, K // gs * gs, gs, bits, seed=M + gs + bits, f16=f16)
+
+
+# 128 x 128 tiles with K split twice at the group sizes that
+# test_qmm_mid_tiles_ragged leaves out and at 8 bits up to 128 rows; five times at
+# group 16.
+@pytest.mark.parametrize("M,N,K,gs,bits", [(500, 3968, 4096, 32, 4), (500, 3968, 4096, 128, 4), (500, 3968, 4096, 32, 8),
+                                           (500, 3968, 4096, 128, 8), (97, 12288, 3072, 64, 8), (955, 768, 5120, 16, 4),
+                                           (955, 768, 5120, 16, 8)])
+def test_qmm_128_row_tiles_split(cuda, M, N, K, gs, bits):
+    run_bounded(M, N, K, gs, bits, seed=M + gs + bits)
+
+
 def at_odd_element(t):
     """t's values at a 2-byte aligned address: element 1 of a larger buffer."""
     flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
@@ -178,11 +207,11 @@ def at_odd_element(t):
 
 
 # Scales and biases at 2-byte addresses (views into one parameter buffer): read
-# two bytes at a time, same values, same sums.  64 x 128 tiles with K split and
-# tails, 96 x 128, 128 x 128 and 128 x 256 tiles.
+# two bytes at a time, same values, same sums.  64 x 128, 96 x 128 and 128 x 128
+# tiles with K split (the last 128 x 256 at group 16) and unsplit 128 x 256 tiles.
 @pytest.mark.parametrize("bits", [4, 8, 6])
 @pytest.mark.parametrize("gs", [16, 32, 64, 128])
-@pytest.mark.parametrize("M,N,K", [(33, 384, 1152), (77, 14336, 512), (130, 256, 256), (600, 3968, 1024)])
+@pytest.mark.parametrize("M,N,K", [(33, 384, 1152), (77, 4224, 2048), (500, 3968, 4096), (1029, 5760, 1280)])
 def test_qmm_parameters_at_two_byte_addresses(cuda, M, N, K, gs, bits):
     print(f"[case] M={M} N={N} K={K} gs={gs} bits={bits}", flush=True)
     w, s, b = device_random_linear(N, K, gs, bits, seed=M + gs + bits)

@@ -123,7 +123,8 @@ def test_gather_widths(cuda, bits, gs, transpose):
 # 2/3/5/6-bit codes re-packed to bytes in the workspace and run by the 8-bit
 # kernel, and group size 16 in that kernel (two groups per lane's 32 codes) --
 # also for 4- and 8-bit codes directly.  N = 384 leaves a partial 256-column
-# tile; M = 17 and 130 partial 128-row tiles; 4096 x 4096 at M = 128 splits K.
+# tile where the planner takes those; M = 17 and 130 partial tiles of rows;
+# 4096 x 4096 at M = 128 splits K.
 PREFILL = [(2, 16, orc.BF16, True), (3, 16, orc.F16, True), (3, 64, orc.BF16, False), (5, 32, orc.F16, True),
            (5, 128, orc.BF16, True), (6, 16, orc.BF16, True), (6, 32, orc.F16, False), (4, 16, orc.BF16, True),
            (8, 16, orc.F16, True)]

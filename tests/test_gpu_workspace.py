@@ -30,7 +30,7 @@ def attn_call(out, q, k, v, kc, vc, freqs, pos, max_seq, st):
 def test_graph_replays_survive_workspace_growth(cuda):
     stream = torch.cuda.Stream()
     st = stream.cuda_stream
-    # split-K prefill (6 tiles on a GPU of 256 CUs: K split several ways)
+    # split-K prefill (20 tiles on a GPU of 256 CUs: K split 4 ways)
     M, N, K = 300, 512, 2048
     w, s, b = synthetic_linear(N, K, 64, 4, seed=1)
     wd, sd, bd = dev_words(w), dev_bf16(s), dev_bf16(b)

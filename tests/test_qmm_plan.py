@@ -57,6 +57,10 @@ def test_parameters_are_read_as_words_only_where_they_are_aligned(rules, gs):
     ((120, 16384, 3072, 128, 8), (64, 128, 1)), ((120, 9216, 2048, 64, 8), (64, 128, 1)),
     ((87, 12160, 5248, 16, 4), (96, 128, 2)), ((128, 10240, 3072, 16, 8), (128, 128, 3)),
     ((955, 768, 13952, 16, 4), (128, 128, 5)), ((300, 1024, 4096, 16, 4), (64, 128, 6)),
+    # the tiles that the GPU tests name
+    ((66, 4224, 2048, 64, 4), (96, 128, 4)), ((96, 5504, 2112, 16, 8), (96, 128, 3)), ((77, 16512, 192, 32, 8), (96, 128, 1)),
+    ((500, 3968, 4096, 128, 8), (128, 128, 2)), ((955, 768, 5120, 16, 8), (128, 128, 5)), ((65, 384, 2048, 64, 4), (64, 128, 4)),
+    ((300, 512, 2048, 64, 8), (64, 128, 4)), ((1029, 5760, 1280, 64, 4), (128, 256, 1)), ((500, 3968, 4096, 16, 4), (128, 256, 4)),
 ])
 def test_tiles_and_splits(rules, shape, tile):
     assert rules.tile(*shape) == tile
