@@ -30,9 +30,12 @@ namespace eq {
 // several passes (a pass multiplies 16 / groups-per-span rows: 8 at 4-bit
 // group 64, 4 at 4-bit group 32, 16 at 8-bit group 64) and the prefill
 // kernel, which reads them once for any M, can take the call (qmm_shape).
-// Measured on the Llama-3-8B shapes: two passes of 4-bit group 64 or of
-// 8-bit group 32 1.0-1.6x slower than the prefill kernel; two passes of
-// 4-bit group 32 within 0.9-1.1x of it, three or more 1.3-2.1x slower.
+// Decode time over that of the prefill kernel (64 x 128 tiles, codes through LDS)
+// on the Llama-3-8B shapes: one pass, up to 8 rows 0.50-0.88, and two of 4-bit
+// group 32 0.67-0.82; two passes of 4-bit group 64 or of 8-bit group 32 0.99-1.48,
+// three or four of 4-bit group 32 1.11-1.56.  One pass of 9 to 16 rows 0.60-0.95 at
+// 4096 rows of weights and fewer; at 14336 and more 0.69-0.88 at 9 rows, 0.95-1.05
+// at 12 and 0.99-1.15 at 16, where the line could lie lower.
 static bool decode_rows(int64_t M, int bits, int group_size, bool qmm_shape) {
     if (M > 16) return false;
     if (!EQ_QMV_ONE_PASS || !qmm_shape) return true;

@@ -495,16 +495,23 @@ unsigned* ws_counters(const WsSource* src, hipStream_t st);
 
 // Routed experts over sorted expert indices (gather_qmm with sorted_indices,
 // transpose, one activation row per route, bf16 x, 4/8-bit, bf16/f16
-// scales): y [batch, N] zeroed, rows x[lhs[b]] gathered into the workspace,
-// a device-built list of (expert, 128-row tile) entries, and one MFMA qmm
-// launch over the list, so each expert's weights are read once per 128
-// routes instead of once per route.  N a multiple of 128, K of 64, x and w
-// 16-byte aligned, y 8-byte aligned.  False (nothing launched) when the
-// workspace cannot be provided or the combination has no kernel.
+// scales): y [batch, N] zeroed, a device-built list of (expert, 64- or 128-row
+// tile) entries in the workspace, and one MFMA qmm launch over the list that
+// reads the rows x[lhs[b]] in place (of 2 GiB of x or more a gathered copy), so
+// each expert's weights are read once per tile instead of once per route.  N a
+// multiple of 128, K of 64, x and w 16-byte aligned, y 8-byte aligned.  False
+// (nothing launched) when the workspace cannot be provided or the combination
+// has no kernel.
 bool launch_qmm_grouped(int bits, int gs, int scale_dtype, uint16_t* y, const uint16_t* x, const uint32_t* w,
                         const void* s, const void* b, const int32_t* lhs, const int32_t* rhs, int batch,
                         int64_t x_batches, int experts, int N, int K, hipStream_t st,
                         const WsSource* src = nullptr);
+
+// Scratch of such a launch over x below 2 GiB, whose rows are read in place (at
+// most): the tile list and its count.
+inline size_t qmm_grouped_list_bytes(int64_t batch, int64_t experts) {
+    return size_t(experts + (batch + 63) / 64 + 1) * 16;
+}
 
 // Everything of eq_gather_qmm after argument validation (gather.hip); `src`
 // (or the stream's workspace when null) holds the grouped path's scratch.

@@ -2145,8 +2145,7 @@ extern "C" int eq_gguf_grouped_linear(void* y, const void* x, const uint8_t* raw
         const size_t wsz = up(size_t(experts * N) * size_t(K) * bits / 8);
         const size_t psz = up(size_t(experts * N) * size_t(K / geo.gs) * 2);
         const size_t triple = wsz + 2 * psz;
-        const int64_t cap = experts + (routes + 127) / 128;  // entries of the grouped tile list
-        const size_t rest = up(size_t(routes) * size_t(K) * 2) + size_t(cap) * 16 + 256;
+        const size_t rest = up(qmm_grouped_list_bytes(routes, experts));
         char* base = static_cast<char*>(ws_acquire(nullptr, triple + rest, st));
         if (!base) {
             set_error("could not obtain workspace for the re-packed expert bank");

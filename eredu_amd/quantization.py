@@ -69,10 +69,8 @@ def _rows(x: torch.Tensor, K: int) -> torch.Tensor:
     return x.reshape(-1, K).contiguous()
 
 
-_MODE_NAME = {}  # QuantizationMode -> its name in bytes, as the C ABI takes it
-
-
-_MODE_NAME.update({m: m.value.encode() for m in QuantizationMode})
+# QuantizationMode -> its name in bytes, as the C ABI takes it
+_MODE_NAME = {m: m.value.encode() for m in QuantizationMode}
 
 
 def _dtype_code(t: torch.Tensor, what: str) -> int:

@@ -204,7 +204,7 @@ int eq_gguf_embedding(void* out, const uint8_t* raw, int64_t raw_len, int ggml_t
  * stay in bounds).  The re-packed bank takes experts * N * (K * b / 8 +
  * 4 * K / gs) bytes of the stream's workspace (b = 4 for Q4_K, 8 for the
  * others; gs = 32, or 16 for Q6_K), every expert whether ids reference it or
- * not, plus routes * K * 2 bytes of gathered rows; the workspace only grows
+ * not, plus 16 bytes per expert and 64 routes; the workspace only grows
  * and is kept until the process ends, so one call on a wide bank holds that
  * memory for the process's lifetime.  Replaces native_grouped_linear (safemlx/src/native_quantization.rs:
  * 1039-1072; its CPU loop :1002-1037) as eredu's MoE calls it
