@@ -14,9 +14,9 @@
 // second K-group adds its sums into the first through LDS.  Wave w of a
 // K-group owns the 64 columns [64w, 64w + 64) and all 128 rows: 4 x 2 tiles of
 // v_mfma_f32_32x32x16_bf16 with f32 accumulators.  Outputs with too few such
-// tiles to fill the GPU without splitting K into short pieces take 128 x 128
-// or 64 x 128 tiles instead (wave w: columns [32w, 32w + 32); the planner,
-// qmm_plan, chooses).
+// tiles to fill the GPU without splitting K into short pieces take 128 x 128,
+// 96 x 128 or 64 x 128 tiles instead (wave w: columns [32w, 32w + 32); the
+// planner, qmm_plan, chooses).
 //
 //  * Everything the loop reads goes straight from memory to LDS
 //    (buffer_load ... lds): a step's activations (two buffers) and its codes
@@ -37,9 +37,10 @@
 //    queue.  One barrier per step, ahead of its last k-step: by then every
 //    wave has read the step's activations and codes, so their buffers can be
 //    refilled, and the next step's have landed, so the next operands can be
-//    prepared under the last MFMAs.  What bounds it now: MFMAs and
-//    dequantization together draw enough power to hold the clock at 1.6-1.9
-//    GHz; at that clock a step takes ~1.3x its MFMAs' cycles.
+//    prepared under the last MFMAs.  What bounds it now: the matrix cores are
+//    busy for 40 % of the cycles at M = 512 and 55 % at M = 4096 (14336 x 4096);
+//    between them the dequantization takes issue slots, and both together hold
+//    the clock at 1.66 GHz with many rows.
 //  * Measured, M = 512, weights rotated from HBM, against two chunks' codes
 //    loaded to registers at the head of each step, the K-groups in opposite
 //    phase and (except group 64) a 2-byte load per parameter: 14336 x 4096
